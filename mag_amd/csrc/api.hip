@@ -35,60 +35,6 @@ int check_dims(mag_ctx c, const int* d) {
 bool is_link(mag_field f) { return f && (f->kind == MAG_LINK18 || f->kind == MAG_LINK12); }
 bool is_alg(mag_field f) { return f && f->kind == MAG_ALG8; }
 
-template <class TS>
-void aos_to_soa(const double* h, TS* s, const Geom& g, int kind) {
-  const int nc = ncomp(kind);
-  if (kind == MAG_REAL1) {
-    for (int site = 0; site < g.V; ++site)
-      for (int mu = 0; mu < 4; ++mu) s[(size_t)mu * g.V + site] = TS(h[(size_t)site * 4 + mu]);
-    return;
-  }
-  const int w = pack_width_rt((int)sizeof(TS), nc);
-  for (int site = 0; site < g.V; ++site)
-    for (int mu = 0; mu < 4; ++mu) {
-      const double* m = h + ((size_t)site * 4 + mu) * 18;
-      if (kind == MAG_ALG8) {
-        M3<double> M;
-        for (int k = 0; k < 9; ++k) M.e[k] = {m[2 * k], m[2 * k + 1]};
-        double a[8];
-        mat_to_alg(M, a);
-        for (int k = 0; k < 8; ++k) s[elem_index(mu, k, site, 8, w, g.V)] = TS(a[k]);
-      } else {
-        for (int k = 0; k < nc; ++k) s[elem_index(mu, k, site, nc, w, g.V)] = TS(m[k]);
-      }
-    }
-}
-
-template <class TS>
-void soa_to_aos(const TS* s, double* h, const Geom& g, int kind) {
-  const int nc = ncomp(kind);
-  if (kind == MAG_REAL1) {
-    for (int site = 0; site < g.V; ++site)
-      for (int mu = 0; mu < 4; ++mu) h[(size_t)site * 4 + mu] = double(s[(size_t)mu * g.V + site]);
-    return;
-  }
-  const int w = pack_width_rt((int)sizeof(TS), nc);
-  for (int site = 0; site < g.V; ++site)
-    for (int mu = 0; mu < 4; ++mu) {
-      double* m = h + ((size_t)site * 4 + mu) * 18;
-      M3<double> M;
-      if (kind == MAG_ALG8) {
-        double a[8];
-        for (int k = 0; k < 8; ++k) a[k] = double(s[elem_index(mu, k, site, 8, w, g.V)]);
-        M = alg_to_mat(a);
-      } else {
-        for (int k = 0; k < nc / 2; ++k)
-          M.e[k] = {double(s[elem_index(mu, 2 * k, site, nc, w, g.V)]),
-                    double(s[elem_index(mu, 2 * k + 1, site, nc, w, g.V)])};
-        if (nc == 12) reconstruct_row2(M);
-      }
-      for (int k = 0; k < 9; ++k) {
-        m[2 * k] = M.e[k].r;
-        m[2 * k + 1] = M.e[k].i;
-      }
-    }
-}
-
 // Device batch for the per-matrix test hooks.
 int batch_hook(mag_ctx c, long n, int prec, const std::vector<const double*>& ins, double* out, int which) {
   if (!c || n < 0 || !out) return MAG_ERR_ARG;
@@ -161,6 +107,7 @@ int mag_ctx_destroy(mag_ctx c) {
   dev_free(c, c->d_scalar, 16 * sizeof(double));
   host_free(c, c->h_scalar, 16 * sizeof(double));
   for (auto e : c->event_pool) (void)hipEventDestroy(e);
+  free_stage(c);
   if (c->owns_stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return MAG_OK;
@@ -262,24 +209,12 @@ int mag_field_info(mag_field f, int dims[4], int* kind, int* prec, size_t* bytes
 
 int mag_field_upload_aos(mag_field f, const double* host) {
   if (!f || !host) return MAG_ERR_ARG;
-  mag_ctx c = f->ctx;
-  std::vector<char> stage(f->bytes);
-  if (f->prec == MAG_F64) aos_to_soa<double>(host, (double*)stage.data(), f->g, f->kind);
-  else aos_to_soa<float>(host, (float*)stage.data(), f->g, f->kind);
-  HIPCHK(c, hipMemcpyAsync(f->p, stage.data(), f->bytes, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  return MAG_OK;
+  return field_transfer(f, const_cast<double*>(host), false);
 }
 
 int mag_field_download_aos(mag_field f, double* host) {
   if (!f || !host) return MAG_ERR_ARG;
-  mag_ctx c = f->ctx;
-  std::vector<char> stage(f->bytes);
-  HIPCHK(c, hipMemcpyAsync(stage.data(), f->p, f->bytes, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (f->prec == MAG_F64) soa_to_aos<double>((const double*)stage.data(), host, f->g, f->kind);
-  else soa_to_aos<float>((const float*)stage.data(), host, f->g, f->kind);
-  return MAG_OK;
+  return field_transfer(f, host, true);
 }
 
 int mag_field_copy(mag_field dst, mag_field src) {

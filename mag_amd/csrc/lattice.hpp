@@ -36,16 +36,6 @@ constexpr int pack_width() {
   constexpr int w = 16 / (int)sizeof(TS);
   return NC % w == 0 ? w : (NC % 2 == 0 ? 2 : 1);
 }
-// Host-side width for a runtime real size and NC (same rule).
-inline int pack_width_rt(int real_bytes, int nc) {
-  if (!MAG_PACK) return 1;
-  const int w = 16 / real_bytes;
-  return nc % w == 0 ? w : (nc % 2 == 0 ? 2 : 1);
-}
-// Index of real c of direction mu at site s (W from pack_width).
-MAG_HD size_t elem_index(int mu, int c, int s, int nc, int w, int V) {
-  return ((size_t)(mu * (nc / w) + c / w) * (size_t)V + (size_t)s) * (size_t)w + (size_t)(c % w);
-}
 
 struct Geom {
   int L[4];

@@ -9,6 +9,7 @@
 
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -76,6 +77,11 @@ struct mag_ctx_s {
   std::vector<hipEvent_t> event_pool;
   mag::Recorder* rec = nullptr;  // set while a serving batch records its launches
   bool owns_stream = true;
+  // pinned slots of host <-> device field transfers (transfer.hip), one transfer at a time
+  std::mutex stage_mu;
+  char* stage = nullptr;
+  size_t stage_cap = 0;
+  std::vector<hipEvent_t> stage_ev;
   std::shared_ptr<mag::MemPool> pool;  // serving child contexts: frees go back to the server's pool
 };
 
@@ -394,6 +400,9 @@ int batch_expiQ(mag_ctx c, const double* dQ, double* dout, long n, int prec);
 int batch_lambda(mag_ctx c, const double* dQ, const double* dS, const double* dU, double* dout, long n, int prec);
 int batch_dexpiq(mag_ctx c, const double* dQ, const double* dDQ, double* dout, long n, int prec);
 double host_uniform(uint64_t seed, uint32_t stream, uint64_t index);
+// transfer.hip: a field's values to (down) or from the qlat layout at `host`
+int field_transfer(mag_field f, double* host, bool down);
+void free_stage(mag_ctx c);
 // noalloc.hip: resolve the allocation-free scratch array of `device` (current)
 int noalloc_setup(int device, std::string* err);
 int constrained_plaq_sum(mag_ctx c, const Geom& g, int prec, int kind, void* U, int mag, int slot, double* norm);

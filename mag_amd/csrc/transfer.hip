@@ -1,0 +1,254 @@
+// Host <-> device movement of fields (mag_field_upload_aos /
+// mag_field_download_aos): the qlat layout on the host ([site][mu][3x3
+// complex], or [site][mu] for one real per link) against the grouped
+// structure-of-arrays in HBM (lattice.hpp).
+//
+// What bounds it: the PCIe link (57 GB/s for a pinned buffer) and the host
+// memory of a fresh user buffer (page faults: 15 GB/s on one thread with
+// huge pages, 50 GB/s on four or more). The conversion itself is done by a
+// kernel that stores the host layout straight into pinned memory (or loads
+// it from there): a block turns 64 sites x 4 directions through LDS, so that
+// its accesses over the link are whole contiguous lines (51-54 GB/s, within
+// 5 % of the DMA engine, without a second copy in HBM). The field goes in
+// chunks through a ring of pinned slots; host threads, two slots each, launch
+// their chunks on the context's stream and copy finished slots to (or fill
+// them from) the caller's buffer, so conversion, link and host copies
+// overlap: 12 ms up and 13-14 ms down (46 GB/s) for any field of 32^4, whose
+// host layout is 604 MB. Converting on one host thread beside a pageable copy
+// of the raw field took 309 / 269 ms for its FP64 links, 106 / 133 ms for the
+// FP32 links and 91 / 101 ms for the momenta.
+//
+// Conversions are the host's own arithmetic (no fused multiply-adds), so the
+// values are bitwise those of a host conversion.
+#pragma clang fp contract(off)
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <exception>
+#include <thread>
+#include <vector>
+
+#include "lattice.hpp"
+#include "runtime.hpp"
+
+using namespace mag;
+
+namespace {
+
+constexpr int TB = 256;           // threads: 64 sites x 4 directions
+constexpr int ROW = 4 * 18;       // doubles per site in the host layout
+constexpr int LROW = ROW + 1;     // LDS row, odd so that the 64 sites of a wave hit different banks
+constexpr size_t CHUNK_MAX = (size_t)4 << 20, CHUNK_MIN = (size_t)512 << 10;
+constexpr int WORKERS_MAX = 4;    // host threads (8 or 12: no faster); 32 MiB of pinned slots at most
+
+typedef double V2 __attribute__((ext_vector_type(2)));
+
+// ALG: eight generator components per link, expanded to (projected from) the 3x3 matrix
+template <class TS, int NC, bool ALG>
+__global__ __launch_bounds__(TB) void k_to_host(TS* p, int V, int s0, int ns, double* out) {
+  __shared__ double buf[64 * LROW];
+  const int lane = threadIdx.x & 63, mu = threadIdx.x >> 6, b0 = blockIdx.x * 64;
+  if (b0 + lane < ns) {
+    TS r[NC];
+    Packed<TS, NC>::template get<NC, true>(p, V, mu, s0 + b0 + lane, r);
+    M3<double> m;
+    if constexpr (ALG) {
+      double h[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) h[k] = double(r[k]);
+      m = alg_to_mat(h);
+    } else {
+#pragma unroll
+      for (int k = 0; k < NC / 2; ++k) m.e[k] = {double(r[2 * k]), double(r[2 * k + 1])};
+      if constexpr (NC == 12) reconstruct_row2(m);
+    }
+    double* b = buf + lane * LROW + mu * 18;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      b[2 * k] = m.e[k].r;
+      b[2 * k + 1] = m.e[k].i;
+    }
+  }
+  __syncthreads();
+  const int n2 = min(64, ns - b0) * (ROW / 2);
+  V2* o = (V2*)(out + (size_t)b0 * ROW);
+  for (int i = threadIdx.x; i < n2; i += TB) {
+    const int site = i / (ROW / 2), c = 2 * (i - site * (ROW / 2));
+    o[i] = V2{buf[site * LROW + c], buf[site * LROW + c + 1]};
+  }
+}
+
+template <class TS, int NC, bool ALG>
+__global__ __launch_bounds__(TB) void k_from_host(TS* p, int V, int s0, int ns, const double* in) {
+  __shared__ double buf[64 * LROW];
+  const int lane = threadIdx.x & 63, mu = threadIdx.x >> 6, b0 = blockIdx.x * 64;
+  const int n2 = min(64, ns - b0) * (ROW / 2);
+  const V2* src = (const V2*)(in + (size_t)b0 * ROW);
+  for (int i = threadIdx.x; i < n2; i += TB) {
+    const int site = i / (ROW / 2), c = 2 * (i - site * (ROW / 2));
+    const V2 v = src[i];
+    buf[site * LROW + c] = v[0];
+    buf[site * LROW + c + 1] = v[1];
+  }
+  __syncthreads();
+  if (b0 + lane >= ns) return;
+  const double* b = buf + lane * LROW + mu * 18;
+  TS r[NC];
+  if constexpr (ALG) {
+    M3<double> m;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) m.e[k] = {b[2 * k], b[2 * k + 1]};
+    double h[8];
+    mat_to_alg(m, h);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) r[k] = TS(h[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < NC; ++k) r[k] = TS(b[k]);
+  }
+  Packed<TS, NC>::template put<false>(p, V, mu, s0 + b0 + lane, r);
+}
+
+// One real per link: [site][mu] on the host, [mu][site] in the field.
+__global__ __launch_bounds__(TB) void k_real_to_host(const double* p, int V, int s0, int ns, double* out) {
+  const int i = blockIdx.x * TB + threadIdx.x;
+  if (i < 4 * ns) out[i] = p[(size_t)(i & 3) * V + s0 + (i >> 2)];
+}
+__global__ __launch_bounds__(TB) void k_real_from_host(double* p, int V, int s0, int ns, const double* in) {
+  const int i = blockIdx.x * TB + threadIdx.x;
+  if (i < 4 * ns) p[(size_t)(i & 3) * V + s0 + (i >> 2)] = in[i];
+}
+
+template <class TS, int NC, bool ALG>
+void launch_matrix(mag_field f, bool down, int s0, int ns, double* slot) {
+  const dim3 grid((ns + 63) / 64);
+  if (down)
+    hipLaunchKernelGGL((k_to_host<TS, NC, ALG>), grid, dim3(TB), 0, f->ctx->stream, (TS*)f->p, f->g.V, s0, ns, slot);
+  else
+    hipLaunchKernelGGL((k_from_host<TS, NC, ALG>), grid, dim3(TB), 0, f->ctx->stream, (TS*)f->p, f->g.V, s0, ns,
+                       (const double*)slot);
+}
+
+// Sites [s0, s0 + ns) of f to (from) a pinned slot.
+hipError_t launch_chunk(mag_field f, bool down, int s0, int ns, double* slot) {
+  const bool f64 = f->prec == MAG_F64;
+  switch (f->kind) {
+    case MAG_REAL1: {
+      const dim3 grid((4 * ns + TB - 1) / TB);
+      if (down)
+        hipLaunchKernelGGL(k_real_to_host, grid, dim3(TB), 0, f->ctx->stream, (const double*)f->p, f->g.V, s0, ns,
+                           slot);
+      else
+        hipLaunchKernelGGL(k_real_from_host, grid, dim3(TB), 0, f->ctx->stream, (double*)f->p, f->g.V, s0, ns,
+                           (const double*)slot);
+      break;
+    }
+    case MAG_ALG8:
+      if (f64) launch_matrix<double, 8, true>(f, down, s0, ns, slot);
+      else launch_matrix<float, 8, true>(f, down, s0, ns, slot);
+      break;
+    case MAG_LINK12:
+      if (f64) launch_matrix<double, 12, false>(f, down, s0, ns, slot);
+      else launch_matrix<float, 12, false>(f, down, s0, ns, slot);
+      break;
+    default:
+      launch_matrix<double, 18, false>(f, down, s0, ns, slot);  // MAG_LINK18 fields are FP64
+  }
+  return hipGetLastError();
+}
+
+// The context's pinned slots and their events, grown to what a call needs.
+int need_stage(mag_ctx c, size_t bytes, size_t events) {
+  if (bytes > c->stage_cap) {
+    if (c->stage) (void)hipHostFree(c->stage);
+    c->stage = nullptr;
+    c->stage_cap = 0;
+    if (hipHostMalloc((void**)&c->stage, bytes, hipHostMallocDefault) != hipSuccess) {
+      c->stage = nullptr;
+      (void)hipGetLastError();
+      return fail(c, MAG_ERR_OOM, "pinned staging allocation failed");
+    }
+    c->stage_cap = bytes;
+  }
+  while (c->stage_ev.size() < events) {
+    hipEvent_t e;
+    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
+      return fail(c, MAG_ERR_DEVICE, "staging event creation failed");
+    c->stage_ev.push_back(e);
+  }
+  return MAG_OK;
+}
+
+}  // namespace
+
+namespace mag {
+
+int field_transfer(mag_field f, double* host, bool down) {
+  mag_ctx c = f->ctx;
+  const std::lock_guard<std::mutex> hold(c->stage_mu);
+  const size_t per = (f->kind == MAG_REAL1 ? 4 : ROW) * sizeof(double), total = per * (size_t)f->g.V;
+  // about eight chunks, 512 KiB (35 GB/s over the link; less is latency) to 4 MiB (50 GB/s) each
+  const size_t want = std::min(std::max(total / 8, CHUNK_MIN), CHUNK_MAX);
+  const int step = (int)((want / per + 63) / 64 * 64);
+  const int nchunk = (f->g.V + step - 1) / step;
+  // one more thread (11 us to start) per 2 MiB: two slots each
+  const int workers = (int)std::min<size_t>({(size_t)WORKERS_MAX, (total + (2 << 20) - 1) / (2 << 20), (size_t)nchunk});
+  const size_t slot_bytes = per * (size_t)std::min(step, f->g.V);
+  int r;
+  if ((r = need_stage(c, slot_bytes * 2 * workers, 2 * (size_t)workers))) return r;
+  std::atomic<int> bad{(int)hipSuccess};
+  std::atomic<int> next{0};
+  auto work = [&](int w) {
+    if (w) (void)hipSetDevice(c->device);  // a new thread starts on device 0
+    char* slot[2] = {c->stage + slot_bytes * (2 * w), c->stage + slot_bytes * (2 * w + 1)};
+    const hipEvent_t ev[2] = {c->stage_ev[2 * w], c->stage_ev[2 * w + 1]};
+    int held[2] = {-1, -1};  // chunk in flight in each slot
+    auto finish = [&](int k) {
+      if (held[k] < 0) return;
+      const hipError_t e = hipEventSynchronize(ev[k]);
+      if (e != hipSuccess) {
+        bad = (int)e;
+      } else if (down) {
+        const size_t s0 = (size_t)held[k] * step, ns = std::min<size_t>(step, f->g.V - s0);
+        std::memcpy((char*)host + s0 * per, slot[k], ns * per);
+      }
+      held[k] = -1;
+    };
+    int k = 0;
+    for (int i = next++; i < nchunk && bad == (int)hipSuccess; i = next++, k ^= 1) {
+      finish(k);
+      const size_t s0 = (size_t)i * step, ns = std::min<size_t>(step, f->g.V - s0);
+      if (!down) std::memcpy(slot[k], (const char*)host + s0 * per, ns * per);
+      hipError_t e = launch_chunk(f, down, (int)s0, (int)ns, (double*)slot[k]);
+      if (e == hipSuccess) {
+        held[k] = i;
+        e = hipEventRecord(ev[k], c->stream);
+      }
+      if (e != hipSuccess) bad = (int)e;
+    }
+    finish(k);
+    finish(k ^ 1);
+  };
+  std::vector<std::thread> pool;
+  try {
+    for (int w = 1; w < workers; ++w) pool.emplace_back(work, w);
+  } catch (const std::exception&) {  // no more threads: those that run take all chunks
+  }
+  work(0);
+  for (auto& t : pool) t.join();
+  if (bad != (int)hipSuccess) {
+    (void)hipStreamSynchronize(c->stream);  // no kernel is left in the slots
+    return fail(c, MAG_ERR_DEVICE, std::string("field transfer: ") + hipGetErrorString((hipError_t)bad.load()));
+  }
+  return MAG_OK;
+}
+
+void free_stage(mag_ctx c) {
+  for (auto e : c->stage_ev) (void)hipEventDestroy(e);
+  c->stage_ev.clear();
+  if (c->stage) (void)hipHostFree(c->stage);
+  c->stage = nullptr;
+  c->stage_cap = 0;
+}
+
+}  // namespace mag
