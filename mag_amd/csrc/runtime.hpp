@@ -238,7 +238,12 @@ inline int fetch_scalars(mag_ctx c, int n) {
 
 inline dim3 grid_links(const Geom& g) { return dim3((g.V + RT_BLOCK - 1) / RT_BLOCK, 4, 1); }
 // Stencil kernels: one 1D tile per (256-site block, mu), see stencil_tile().
-inline dim3 grid_stencil(const Geom& g) { return dim3(4 * ((g.V + RT_BLOCK - 1) / RT_BLOCK), 1, 1); }
+// The grid is rounded up to whole rounds over the 8 XCDs (the last few blocks
+// hold no sites): with a remainder the tiles would go to the XCDs one by one
+// instead of in contiguous runs, and share no neighbours in L2. Iwasaki +
+// 3-stout force: 20^4 FP64 1735 -> 1254 us, FP32 687 -> 550; 14^4 510 -> 378,
+// 196 -> 179.
+inline dim3 grid_stencil(const Geom& g) { return dim3((4 * ((g.V + RT_BLOCK - 1) / RT_BLOCK) + 7) / 8 * 8, 1, 1); }
 
 // ------------------------------------------------------------ workspace
 // Scratch of one lattice shape and storage format, owned by the context and
