@@ -32,16 +32,12 @@ constexpr int BLOCK = 256;
 // the Iwasaki top kernel 20 %). FP64 stout kernels are held to 2 waves:
 // unbounded they take 256 VGPRs plus 4-20 AGPRs and run 1 wave; at 2 waves
 // they spill 20-116 bytes per lane and the backward and top kernels ran 16 %
-// and 9 % faster. The FP64 thin-link force runs at 1 wave without spills: at
-// 2 it spilled 116 bytes (free links) or 536 (constraint classes) and was 6 %
-// slower on the grouped layout (the top kernel, with the same staple sum,
-// runs equally fast at 1 and 2 waves there).
+// and 9 % faster.
 template <class TC>
 constexpr int stencil_waves() { return sizeof(TC) == sizeof(float) ? 3 : 2; }
-template <class TC, bool CONS>
-constexpr int gforce_waves() { return sizeof(TC) == sizeof(float) ? 3 : 1; }
 #define MAG_STENCIL_OCC __attribute__((amdgpu_waves_per_eu(stencil_waves<TC>())))
-#define MAG_GFORCE_OCC __attribute__((amdgpu_waves_per_eu(gforce_waves<TC, CONS>())))
+// FP64 thin-link force: 1 wave without spills (constrained rectangles spill 536 bytes at 2)
+#define MAG_GFORCE_OCC __attribute__((amdgpu_waves_per_eu(sizeof(TC) == sizeof(float) ? 3 : 1)))
 
 // Blocks are dispatched round-robin over the 8 XCDs (XCD = linear block id
 // mod 8). When L3 splits into 8 slabs and an x3 slice is a whole number of
@@ -58,12 +54,12 @@ constexpr int gforce_waves() { return sizeof(TC) == sizeof(float) ? 3 : 1; }
 // order). Otherwise XCD k takes tiles [k nb/8, (k+1) nb/8) in lexicographic
 // order. nb = blocks in the launch, b = this block; every (mu, sblk) of the
 // 4 V / BLOCK tiles comes out of exactly one b.
-template <bool X2_INNER = false>
+template <bool X2_INNER = false, int BS = BLOCK>
 MAG_HD void tile_map(const Geom& g, int nb, int b, int& mu, int& sblk) {
   const int plane = g.L[0] * g.L[1];
   const int slice = plane * g.L[2];
-  const bool slab = nb % 8 == 0 && g.L[3] % 8 == 0 && nb == 4 * (g.V / BLOCK) &&
-                    (X2_INNER ? plane % BLOCK == 0 : slice % BLOCK == 0);
+  const bool slab = nb % 8 == 0 && g.L[3] % 8 == 0 && nb == 4 * (g.V / BS) &&
+                    (X2_INNER ? plane % BS == 0 : slice % BS == 0);
   if (slab) {
     const int xcd = b % 8, j = b / 8;
     const int h3 = g.L[3] / 8;
@@ -73,14 +69,14 @@ MAG_HD void tile_map(const Geom& g, int nb, int b, int& mu, int& sblk) {
     r /= h3;
     int bs;  // block within the x3 slice
     if (X2_INNER) {
-      const int nb01 = plane / BLOCK;
+      const int nb01 = plane / BS;
       const int x2 = r % g.L[2];
       bs = x2 * nb01 + r / g.L[2];
     } else {
       bs = r;
     }
     const int x3 = xcd * h3 + dx3;
-    sblk = x3 * (slice / BLOCK) + bs;
+    sblk = x3 * (slice / BS) + bs;
     return;
   }
   const int t = (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;
@@ -92,6 +88,81 @@ MAG_D void stencil_tile(const Geom& g, int& mu, int& sblk) {
   tile_map<X2_INNER>(g, gridDim.x, blockIdx.x, mu, sblk);
 }
 
+// ---- stencils by planes (split form)
+// What a stencil kernel sums at a link falls into three shares, one per plane
+// through it. The split form gives each plane a wavefront of its own: a block
+// is 64 sites of one direction by three wavefronts, which sum their shares in
+// LDS in plane order, and the first of them goes on alone with what follows
+// the sum. Rules and measurements at launch_stencil().
+//
+// A stencil K has Args (with Geom g), Real, waves (per SIMD),
+// share(args, site, mu, plane) and finish(args, mu, s, sum).
+constexpr int PLANE_SITES = 64, PLANE_THREADS = 3 * PLANE_SITES;
+
+template <class TC>
+MAG_D void share_put(TC* red, int slot, const M3<TC>& S) {
+  TC* r = red + slot * 18 * 64 + (threadIdx.x & 63);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {
+    r[2 * k * 64] = S.e[k].r;
+    r[(2 * k + 1) * 64] = S.e[k].i;
+  }
+}
+template <class TC>
+MAG_D void share_add(const TC* red, int slot, M3<TC>& S) {
+  const TC* r = red + slot * 18 * 64 + (threadIdx.x & 63);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) S.e[k] = {S.e[k].r + r[2 * k * 64], S.e[k].i + r[(2 * k + 1) * 64]};
+}
+MAG_D int wave_of_block() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }  // a scalar register
+
+// The 64-site groups of XCD k (block id mod 8), walked by i; -1 past the end.
+// With whole-group slices and L3 in 8 slabs of 3 or more the order of
+// tile_map (x3 of the slab fastest, then x2, then the rest of the slice):
+// FP64 top kernel at 32^4 2.08-2.16 ms against 2.45. Otherwise groups
+// [k n/8, (k+1) n/8) in site order: at 16^4, whose slabs are two slices, 137
+// against 143 us.
+MAG_HD int plane_group(const Geom& g, int xcd, int i) {
+  const int n = (g.V + PLANE_SITES - 1) / PLANE_SITES;
+  const int lo = (int)((long)n * xcd / 8), hi = (int)((long)n * (xcd + 1) / 8);
+  if (i >= hi - lo) return -1;
+  const int plane = g.L[0] * g.L[1], slice = plane * g.L[2];
+  if (g.L[3] % 8 == 0 && g.L[3] >= 24 && slice % PLANE_SITES == 0) {
+    const int h3 = g.L[3] / 8, x3 = xcd * h3 + i % h3;
+    int r = i / h3;  // group of the slice
+    if (plane % PLANE_SITES == 0) r = (r % g.L[2]) * (plane / PLANE_SITES) + r / g.L[2];
+    return x3 * (slice / PLANE_SITES) + r;
+  }
+  return lo + i;
+}
+
+// Block b of a split stencil, with two slots of LDS at red.
+template <class K>
+MAG_D void split_block(const typename K::Args& a, int b, typename K::Real* red) {
+  using TC = typename K::Real;
+  const int xcd = b & 7, j = b >> 3, mu = j & 3, plane = wave_of_block();
+  const int grp = plane_group(a.g, xcd, j >> 2);
+  if (grp < 0) return;
+  const int s = grp * PLANE_SITES + (threadIdx.x & 63);
+  M3<TC> S = K::share(a, site_of(a.g, min(s, a.g.V - 1)), mu, plane);
+  if (plane > 0) share_put(red, plane - 1, S);
+  __syncthreads();
+  if (plane > 0) return;
+  share_add(red, 0, S);
+  share_add(red, 1, S);
+  if (s < a.g.V) K::finish(a, mu, s, S);
+}
+template <class K>
+MAG_D void split_body(const typename K::Args& a) {
+  __shared__ typename K::Real red[2 * 18 * 64];
+  split_block<K>(a, blockIdx.x, red);
+}
+template <class K>
+__global__ __launch_bounds__(PLANE_THREADS) __attribute__((amdgpu_waves_per_eu(K::waves))) void k_split(
+    typename K::Args a) { split_body<K>(a); }
+template <class K>
+__global__ __launch_bounds__(PLANE_THREADS) __attribute__((amdgpu_waves_per_eu(K::waves))) void k_split_b(
+    const typename K::Args* t) { split_body<K>(t[blockIdx.z]); }
 // ======================================================= staples and forces
 enum ActionKind : int { ACT_WILSON = 0, ACT_IWASAKI = 1 };
 
@@ -219,6 +290,23 @@ MAG_D M3<TC> staple_sum_nav(const UV& u, const NAV& nv, int mu, TC c0, TC c1) {
   return S;
 }
 
+// The share of the staple sum that plane i of the three gives.
+template <int ACT, class TC, class UV>
+MAG_D M3<TC> staple_share(const UV& u, const Geom& g, const Site& p, int mu, int i, TC c0, TC c1) {
+  const GNav nv{g, p};
+  M3<TC> S = zero3<TC>();
+  M3<TC> R = zero3<TC>();
+  const auto xpm = nv.at() + nv.off(mu, 1);
+  const auto xmm = nv.at() + nv.off(mu, -1);
+  const auto xp2m = nv.at() + nv.off(mu, 2);
+  staple_plane<ACT, TC>(u, nv, mu, i + (i >= mu ? 1 : 0), xpm, xmm, xp2m, c0, c1, S, R);
+  if (ACT == ACT_IWASAKI) {
+    R = scale(R, c1);
+    mul_nd_acc(S, R, u.template load<TC>(mu, xpm));
+  }
+  return S;
+}
+
 template <int ACT, class TS, int NC, class TC>
 MAG_D M3<TC> staple_sum(const LinkView<TS, NC>& u, const Geom& g, const Site& p, int mu, TC c0, TC c1) {
   return staple_sum_nav<ACT, TC>(u, GNav{g, p}, mu, c0, c1);
@@ -242,6 +330,7 @@ struct ForceArgs {
   int mag;
   int out;
   double eps;
+  int npair;  // k_cons_force: blocks of links with two staple sums
 };
 
 template <class TS, int NC, class TC>
@@ -264,12 +353,34 @@ MAG_D void force_epilogue(const ForceArgs<TS, NC>& a, int mu, int s, const M3<TC
   }
 }
 
+// F_a = -(beta/3) Im Tr(T_a W) into the chosen output.
+template <class TS, int NC, class TC>
+MAG_D void gauge_force_link(const ForceArgs<TS, NC>& a, int mu, int s, const M3<TC>& Ux, const M3<TC>& W) {
+  TC f[8];
+  force_alg_from(W, f);
+  const TC fac = TC(-a.beta / 3.);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) f[k] *= fac;
+  force_epilogue<TS, NC, TC>(a, mu, s, Ux, f);
+}
+
 // get_force (field-hmc.h:339-425): F = (i beta/3) TA(W) with W = U S^+ for
 // free links, W = U(x+mu) S(x+mu)^+ - S(x)^+ U(x) for constraint classes 1 and
 // 10, and F = 0 for class 100. Stored as F_a = -(beta/3) Im Tr(T_a W).
-// CONS = false (mag = 0) compiles the free-link form alone (one staple sum,
-// no class loop, U(x) loaded after it).
-template <int ACT, bool CONS, class TS, int NC, class TC, bool R12 = false>
+// In the split form (CONS) a block forms one staple sum for every link and
+// leaves out classes 1 and 10, 1/16 of the links at mag = 2, which
+// k_cons_force gathers in blocks of their own with their two sums.
+template <bool CONS, class TS, int NC, class TC>
+MAG_D void force_link(const ForceArgs<TS, NC>& a, const Site& p, int mu, const M3<TC>& S) {
+  const int cls = CONS ? link_class_rt(p, mu, a.mag) : 0;
+  if (cls == 1 || cls == 10) return;
+  const M3<TC> Ux = a.U.template load<TC>(mu, p.s);
+  M3<TC> W = mul_nd(Ux, S);
+  if (cls == 100) W = zero3<TC>();
+  gauge_force_link<TS, NC, TC>(a, mu, p.s, Ux, W);
+}
+// One thread per link; constrained links of classes 1 and 10 walk both sums.
+template <int ACT, bool CONS, class TS, int NC, class TC>
 MAG_D void k_gauge_force_body(const ForceArgs<TS, NC>& a) {
   int mu, sblk;
   stencil_tile<sizeof(TC) == sizeof(double)>(a.g, mu, sblk);
@@ -281,14 +392,12 @@ MAG_D void k_gauge_force_body(const ForceArgs<TS, NC>& a) {
   M3<TC> Ux, W = zero3<TC>();
   if (!CONS) {
     // U(x) is loaded after the staple sum, so it is not live across it
-    M3<TC> S;
-    if constexpr (R12) S = staple_sum_nav<ACT, TC>(SU3Read<TS, NC>{a.U}, GNav{a.g, p}, mu, c0, c1);
-    else S = staple_sum<ACT, TS, NC, TC>(a.U, a.g, p, mu, c0, c1);
-    Ux = a.U.template load_su3<TC, R12>(mu, s);
+    const M3<TC> S = staple_sum<ACT, TS, NC, TC>(a.U, a.g, p, mu, c0, c1);
+    Ux = a.U.template load<TC>(mu, s);
     W = mul_nd(Ux, S);
   } else {
     const int cls = link_class_rt(p, mu, a.mag);
-    Ux = a.U.template load_su3<TC, R12>(mu, s);
+    Ux = a.U.template load<TC>(mu, s);
     if (cls != 100) {
       // class 0: one staple at x; classes 1, 10: staples at x and x+mu
       const int nsite = (cls == 0) ? 1 : 2;
@@ -296,26 +405,93 @@ MAG_D void k_gauge_force_body(const ForceArgs<TS, NC>& a) {
 #pragma unroll 1
       for (int k = 0; k < nsite; ++k) {
         const Site q = (k == 0) ? p : site_of(a.g, ys);
-        M3<TC> S;
-        if constexpr (R12) S = staple_sum_nav<ACT, TC>(SU3Read<TS, NC>{a.U}, GNav{a.g, q}, mu, c0, c1);
-        else S = staple_sum<ACT, TS, NC, TC>(a.U, a.g, q, mu, c0, c1);
+        const M3<TC> S = staple_sum<ACT, TS, NC, TC>(a.U, a.g, q, mu, c0, c1);
         if (cls == 0) W = mul_nd(Ux, S);
         else if (k == 0) W = sub(W, mul_dn(S, Ux));
-        else mul_nd_acc(W, a.U.template load_su3<TC, R12>(mu, ys), S);
+        else mul_nd_acc(W, a.U.template load<TC>(mu, ys), S);
       }
     }
   }
-  TC f[8];
-  force_alg_from(W, f);
-  const TC fac = TC(-a.beta / 3.);
-#pragma unroll
-  for (int k = 0; k < 8; ++k) f[k] *= fac;
-  force_epilogue<TS, NC, TC>(a, mu, s, Ux, f);
+  gauge_force_link<TS, NC, TC>(a, mu, s, Ux, W);
 }
-template <int ACT, bool CONS, class TS, int NC, class TC, bool R12 = false>
-__global__ __launch_bounds__(BLOCK) MAG_GFORCE_OCC void k_gauge_force(ForceArgs<TS, NC> a) { k_gauge_force_body<ACT, CONS, TS, NC, TC, R12>(a); }
-template <int ACT, bool CONS, class TS, int NC, class TC, bool R12 = false>
-__global__ __launch_bounds__(BLOCK) MAG_GFORCE_OCC void k_gauge_force_b(const ForceArgs<TS, NC>* t) { k_gauge_force_body<ACT, CONS, TS, NC, TC, R12>(t[blockIdx.z]); }
+template <int ACT, bool CONS, class TS, int NC, class TC>
+__global__ __launch_bounds__(BLOCK) MAG_GFORCE_OCC void k_gauge_force(ForceArgs<TS, NC> a) { k_gauge_force_body<ACT, CONS, TS, NC, TC>(a); }
+template <int ACT, bool CONS, class TS, int NC, class TC>
+__global__ __launch_bounds__(BLOCK) MAG_GFORCE_OCC void k_gauge_force_b(const ForceArgs<TS, NC>* t) { k_gauge_force_body<ACT, CONS, TS, NC, TC>(t[blockIdx.z]); }
+
+template <int ACT, bool CONS, class TS, int NC, class TC>
+struct ForceStencil {
+  using Args = ForceArgs<TS, NC>;
+  using Real = TC;
+  static constexpr int waves = stencil_waves<TC>();
+  MAG_D static M3<TC> share(const Args& a, const Site& p, int mu, int plane) {
+    const TC c1 = (ACT == ACT_IWASAKI) ? TC(a.c1) : TC(0);
+    return staple_share<ACT, TC>(a.U, a.g, p, mu, plane, TC(1) - TC(8) * c1, c1);
+  }
+  MAG_D static void finish(const Args& a, int mu, int s, const M3<TC>& S) {
+    force_link<CONS, TS, NC, TC>(a, site_of(a.g, s), mu, S);
+  }
+};
+
+// Links of direction mu of classes 1 and 10: transverse coordinates multiples
+// of mag, the own coordinate not the last of its block.
+MAG_HD int pair_count(const Geom& g, int mu, int mag) {
+  const int Lm = sel4(g.L, mu);
+  int n = (Lm / mag) * (mag - 1) + Lm % mag;
+  for (int i = 0; i < 4; ++i)
+    if (i != mu) n *= (g.L[i] + mag - 1) / mag;
+  return n;
+}
+MAG_HD Site pair_site(const Geom& g, int mu, int mag, int t) {
+  Site p;
+  p.s = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int n = i == mu ? (g.L[i] / mag) * (mag - 1) + g.L[i] % mag : (g.L[i] + mag - 1) / mag;
+    const int h = t % n;
+    t /= n;
+    p.x[i] = i == mu ? h / (mag - 1) * mag + h % (mag - 1) : h * mag;
+    p.s += p.x[i] * g.S[i];
+  }
+  return p;
+}
+// Thin force of a constrained run on a small lattice: first the blocks of
+// those links, 64 of one direction each, a wavefront per plane that forms its
+// share of both sums; then the blocks of the split stencil.
+template <int ACT, class TS, int NC, class TC>
+MAG_D void k_cons_force_body(const ForceArgs<TS, NC>& a) {
+  __shared__ TC red[5 * 18 * 64];  // shares of S(x) in slots 0-2, planes 1 and 2 of S(x+mu) in 3, 4
+  if ((int)blockIdx.x >= a.npair) {
+    split_block<ForceStencil<ACT, true, TS, NC, TC>>(a, (int)blockIdx.x - a.npair, red);
+    return;
+  }
+  const int mu = blockIdx.x & 3, plane = wave_of_block();
+  const int n = pair_count(a.g, mu, a.mag), t0 = (blockIdx.x >> 2) * 64, t = t0 + (threadIdx.x & 63);
+  if (t0 >= n) return;
+  const TC c1 = (ACT == ACT_IWASAKI) ? TC(a.c1) : TC(0), c0 = TC(1) - TC(8) * c1;
+  const Site p = pair_site(a.g, mu, a.mag, min(t, n - 1));
+  const Site q = site_of(a.g, p.s + off_rt(a.g, p, mu, 1));
+  M3<TC> S;
+#pragma unroll 1
+  for (int k = 0; k < 2; ++k) {
+    S = staple_share<ACT, TC>(a.U, a.g, k ? q : p, mu, plane, c0, c1);
+    if (k == 0 || plane > 0) share_put(red, k ? 2 + plane : plane, S);
+  }
+  __syncthreads();
+  if (plane > 0 || t >= n) return;
+  share_add(red, 3, S);
+  share_add(red, 4, S);
+  M3<TC> W = mul_nd(a.U.template load<TC>(mu, q.s), S);
+  S = zero3<TC>();
+  for (int k = 0; k < 3; ++k) share_add(red, k, S);
+  const M3<TC> Ux = a.U.template load<TC>(mu, p.s);
+  W = sub(W, mul_dn(S, Ux));
+  gauge_force_link<TS, NC, TC>(a, mu, p.s, Ux, W);
+}
+template <int ACT, class TS, int NC, class TC>
+__global__ __launch_bounds__(PLANE_THREADS) MAG_STENCIL_OCC void k_cons_force(ForceArgs<TS, NC> a) { k_cons_force_body<ACT, TS, NC, TC>(a); }
+template <int ACT, class TS, int NC, class TC>
+__global__ __launch_bounds__(PLANE_THREADS) MAG_STENCIL_OCC void k_cons_force_b(const ForceArgs<TS, NC>* t) { k_cons_force_body<ACT, TS, NC, TC>(t[blockIdx.z]); }
 
 // ============================================================ link updates
 // evolve_gauge_field (field-hmc.h:442-482) with the constraint classes:
@@ -411,16 +587,9 @@ struct StoutFwdArgs {
   int store_qc;  // 0 when only the smeared field is wanted (Hamiltonian)
 };
 
-template <class TSI, int NCI, class TSO, int NCO, class TC, bool R12 = false>
-MAG_D void k_stout_fwd_body(const StoutFwdArgs<TSI, NCI, TSO, NCO>& a) {
-  int mu, sblk;
-  stencil_tile(a.g, mu, sblk);
-  const int s = sblk * BLOCK + threadIdx.x;
-  if (s >= a.g.V) return;
-  const Site p = site_of(a.g, s);
-  M3<TC> S;
-  if constexpr (R12) S = staple_sum_nav<ACT_WILSON, TC>(SU3Read<TSI, NCI>{a.U}, GNav{a.g, p}, mu, TC(1), TC(0));
-  else S = staple_sum<ACT_WILSON, TSI, NCI, TC>(a.U, a.g, p, mu, TC(1), TC(0));
+// Q, C and the smeared link from the link's staple sum S.
+template <class TSI, int NCI, class TSO, int NCO, class TC, bool R12>
+MAG_D void stout_fwd_link(const StoutFwdArgs<TSI, NCI, TSO, NCO>& a, int mu, int s, const M3<TC>& S) {
   const M3<TC> Ux = a.U.template load_su3<TC, R12>(mu, s);
   TC q[8];
   force_alg_from(mul_nd(S, Ux), q);  // -i TA(S U^+)
@@ -435,9 +604,35 @@ MAG_D void k_stout_fwd_body(const StoutFwdArgs<TSI, NCI, TSO, NCO>& a) {
   }
 }
 template <class TSI, int NCI, class TSO, int NCO, class TC, bool R12 = false>
+MAG_D void k_stout_fwd_body(const StoutFwdArgs<TSI, NCI, TSO, NCO>& a) {
+  int mu, sblk;
+  stencil_tile(a.g, mu, sblk);
+  const int s = sblk * BLOCK + threadIdx.x;
+  if (s >= a.g.V) return;
+  const Site p = site_of(a.g, s);
+  M3<TC> S;
+  if constexpr (R12) S = staple_sum_nav<ACT_WILSON, TC>(SU3Read<TSI, NCI>{a.U}, GNav{a.g, p}, mu, TC(1), TC(0));
+  else S = staple_sum<ACT_WILSON, TSI, NCI, TC>(a.U, a.g, p, mu, TC(1), TC(0));
+  stout_fwd_link<TSI, NCI, TSO, NCO, TC, R12>(a, mu, s, S);
+}
+template <class TSI, int NCI, class TSO, int NCO, class TC, bool R12 = false>
 __global__ __launch_bounds__(BLOCK) MAG_STENCIL_OCC void k_stout_fwd(StoutFwdArgs<TSI, NCI, TSO, NCO> a) { k_stout_fwd_body<TSI, NCI, TSO, NCO, TC, R12>(a); }
 template <class TSI, int NCI, class TSO, int NCO, class TC, bool R12 = false>
 __global__ __launch_bounds__(BLOCK) MAG_STENCIL_OCC void k_stout_fwd_b(const StoutFwdArgs<TSI, NCI, TSO, NCO>* t) { k_stout_fwd_body<TSI, NCI, TSO, NCO, TC, R12>(t[blockIdx.z]); }
+
+template <class TSI, int NCI, class TSO, int NCO, class TC, bool R12 = false>
+struct FwdStencil {
+  using Args = StoutFwdArgs<TSI, NCI, TSO, NCO>;
+  using Real = TC;
+  static constexpr int waves = stencil_waves<TC>();
+  MAG_D static M3<TC> share(const Args& a, const Site& p, int mu, int plane) {
+    if constexpr (R12) return staple_share<ACT_WILSON, TC>(SU3Read<TSI, NCI>{a.U}, a.g, p, mu, plane, TC(1), TC(0));
+    else return staple_share<ACT_WILSON, TC>(a.U, a.g, p, mu, plane, TC(1), TC(0));
+  }
+  MAG_D static void finish(const Args& a, int mu, int s, const M3<TC>& S) {
+    stout_fwd_link<TSI, NCI, TSO, NCO, TC, R12>(a, mu, s, S);
+  }
+};
 
 // Lambda step of level k for one link, given Z' = dS/dU_{k+1} there
 // (compute_Lambda, field-multi.h:180-269, eqs. 72-73):
@@ -478,10 +673,7 @@ struct StoutTopArgs {
   double beta, c1, rho;
 };
 
-// R12: the staple links of U_n (and U_{n-1}) read as rows 0 and 1 with row 2
-// rebuilt; such a kernel runs at one wave per SIMD (its spills then go to
-// AGPRs, not scratch).
-template <int ACT, class TS, int NC, class TC, int NCN, bool R12 = false>
+template <int ACT, class TS, int NC, class TC, int NCN>
 MAG_D void k_stout_top_body(const StoutTopArgs<TS, NC, NCN>& a) {
   int mu, sblk;
   stencil_tile<sizeof(TC) == sizeof(double)>(a.g, mu, sblk);
@@ -490,23 +682,31 @@ MAG_D void k_stout_top_body(const StoutTopArgs<TS, NC, NCN>& a) {
   const TC c1 = (ACT == ACT_IWASAKI) ? TC(a.c1) : TC(0);
   const TC c0 = TC(1) - TC(8) * c1;
   const Site p = site_of(a.g, s);
-  M3<TC> S;
-  if constexpr (R12) S = staple_sum_nav<ACT, TC>(SU3Read<TS, NCN>{a.Un}, GNav{a.g, p}, mu, c0, c1);
-  else S = staple_sum<ACT, TS, NCN, TC>(a.Un, a.g, p, mu, c0, c1);
+  const M3<TC> S = staple_sum<ACT, TS, NCN, TC>(a.Un, a.g, p, mu, c0, c1);
   const M3<TC> Z = scale(dag(S), TC(-a.beta / 3.));
-  stout_lambda_link<TS, NC, TC, R12>(mu, s, Z, a.Ulo, a.Qlo, a.Clo, a.Lout, a.Wout);
+  stout_lambda_link<TS, NC, TC>(mu, s, Z, a.Ulo, a.Qlo, a.Clo, a.Lout, a.Wout);
 }
-template <class TC, bool R12>
-constexpr int top_waves() { return R12 ? 1 : stencil_waves<TC>(); }
-template <int ACT, class TS, int NC, class TC, int NCN = NC, bool R12 = false>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(top_waves<TC, R12>()))) void k_stout_top(
-    StoutTopArgs<TS, NC, NCN> a) {
-  k_stout_top_body<ACT, TS, NC, TC, NCN, R12>(a);
+template <int ACT, class TS, int NC, class TC, int NCN = NC>
+struct TopStencil {
+  using Args = StoutTopArgs<TS, NC, NCN>;
+  using Real = TC;
+  static constexpr int waves = stencil_waves<TC>();
+  MAG_D static M3<TC> share(const Args& a, const Site& p, int mu, int plane) {
+    const TC c1 = (ACT == ACT_IWASAKI) ? TC(a.c1) : TC(0);
+    return staple_share<ACT, TC>(a.Un, a.g, p, mu, plane, TC(1) - TC(8) * c1, c1);
+  }
+  MAG_D static void finish(const Args& a, int mu, int s, const M3<TC>& S) {
+    stout_lambda_link<TS, NC, TC>(mu, s, scale(dag(S), TC(-a.beta / 3.)), a.Ulo, a.Qlo, a.Clo, a.Lout, a.Wout);
+  }
+};
+
+template <int ACT, class TS, int NC, class TC, int NCN = NC>
+__global__ __launch_bounds__(BLOCK) MAG_STENCIL_OCC void k_stout_top(StoutTopArgs<TS, NC, NCN> a) {
+  k_stout_top_body<ACT, TS, NC, TC, NCN>(a);
 }
-template <int ACT, class TS, int NC, class TC, int NCN = NC, bool R12 = false>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(top_waves<TC, R12>()))) void k_stout_top_b(
-    const StoutTopArgs<TS, NC, NCN>* t) {
-  k_stout_top_body<ACT, TS, NC, TC, NCN, R12>(t[blockIdx.z]);
+template <int ACT, class TS, int NC, class TC, int NCN = NC>
+__global__ __launch_bounds__(BLOCK) MAG_STENCIL_OCC void k_stout_top_b(const StoutTopArgs<TS, NC, NCN>* t) {
+  k_stout_top_body<ACT, TS, NC, TC, NCN>(t[blockIdx.z]);
 }
 
 // ---- LDS-tiled variant of the FP32 Iwasaki top kernel (MAG_TOP_LDS).
@@ -699,57 +899,60 @@ MAG_HD void mul_nd_sub(M3<T>& c, const M3<T>& a, const M3<T>& b) {
     }
 }
 
+// The two terms of the plane (mu, nu), without the factor i rho.
 template <class TS, int NC, class TC, bool R12>
-MAG_D M3<TC> stout_six_terms(const StoutBwdArgs<TS, NC>& a, const Site& p, int mu) {
+MAG_D void stout_plane(const StoutBwdArgs<TS, NC>& a, const Site& p, int mu, int nu, int xpm, M3<TC>& acc) {
   const Geom& g = a.g;
-  M3<TC> acc = zero3<TC>();
-  const int xpm = p.s + off_rt(g, p, mu, 1);
-#pragma unroll 1
-  for (int i = 0; i < 3; ++i) {
-    const int nu = i + (i >= mu ? 1 : 0);
-    const int opn = off_rt(g, p, nu, 1), omn = off_rt(g, p, nu, -1);
-    const int xpn = p.s + opn, xmn = p.s + omn, xpmmn = xpm + omn;
-    {
-      // D and E = D U_nu(x)^+ are products of links: formed in two rows, completed once
-      M3<TC> D = mul_nd_r2(a.U.template load_r2<TC>(nu, xpm), a.U.template load_su3<TC, R12>(mu, xpn));
-      reconstruct_row2(D);
-      M3<TC> G = mul_hn(a.L.template load_mat<TC>(nu, xpm), D);
-      mul_sub_nh(G, D, a.L.template load_mat<TC>(mu, xpn));
-      const M3<TC> Un_x = a.U.template load_su3<TC, R12>(nu, p.s);
-      mul_nd_acc(acc, G, Un_x);
-      M3<TC> E = mul_nd_r2(D, Un_x);
-      reconstruct_row2(E);
-      mul_sub_nh(acc, E, a.L.template load_mat<TC>(nu, p.s));
-    }
-    {
-      const M3<TC> Um_xmn = a.U.template load_su3<TC, R12>(mu, xmn);
-      TC ln[8], lm[8];
-      a.L.load(nu, xmn, ln);
-      a.L.load(mu, xmn, lm);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) ln[k] -= lm[k];
-      M3<TC> K = mul_dh(Um_xmn, alg_to_mat(ln));
-      mul_hd_sub(K, a.L.template load_mat<TC>(nu, xpmmn), Um_xmn);
-      const M3<TC> K2 = mul_dn(a.U.template load_su3<TC, R12>(nu, xpmmn), K);
-      mul_acc(acc, K2, a.U.template load_su3<TC, R12>(nu, xmn));
-    }
+  const int opn = off_rt(g, p, nu, 1), omn = off_rt(g, p, nu, -1);
+  const int xpn = p.s + opn, xmn = p.s + omn, xpmmn = xpm + omn;
+  {
+    // D and E = D U_nu(x)^+ are products of links: formed in two rows, completed once
+    M3<TC> D = mul_nd_r2(a.U.template load_r2<TC>(nu, xpm), a.U.template load_su3<TC, R12>(mu, xpn));
+    reconstruct_row2(D);
+    M3<TC> G = mul_hn(a.L.template load_mat<TC>(nu, xpm), D);
+    mul_sub_nh(G, D, a.L.template load_mat<TC>(mu, xpn));
+    const M3<TC> Un_x = a.U.template load_su3<TC, R12>(nu, p.s);
+    mul_nd_acc(acc, G, Un_x);
+    M3<TC> E = mul_nd_r2(D, Un_x);
+    reconstruct_row2(E);
+    mul_sub_nh(acc, E, a.L.template load_mat<TC>(nu, p.s));
   }
-  // Z = W + i rho acc
-  M3<TC> Z = a.W.template load_nt<TC>(mu, p.s);
+  {
+    const M3<TC> Um_xmn = a.U.template load_su3<TC, R12>(mu, xmn);
+    TC ln[8], lm[8];
+    a.L.load(nu, xmn, ln);
+    a.L.load(mu, xmn, lm);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) ln[k] -= lm[k];
+    M3<TC> K = mul_dh(Um_xmn, alg_to_mat(ln));
+    mul_hd_sub(K, a.L.template load_mat<TC>(nu, xpmmn), Um_xmn);
+    const M3<TC> K2 = mul_dn(a.U.template load_su3<TC, R12>(nu, xpmmn), K);
+    mul_acc(acc, K2, a.U.template load_su3<TC, R12>(nu, xmn));
+  }
+}
+
+// Z = W + i rho acc
+template <class TS, int NC, class TC>
+MAG_D M3<TC> stout_Z(const StoutBwdArgs<TS, NC>& a, int mu, int s, const M3<TC>& acc) {
+  M3<TC> Z = a.W.template load_nt<TC>(mu, s);
   const TC rho = TC(a.rho);
 #pragma unroll
   for (int k = 0; k < 9; ++k) Z.e[k] = {mfma(-rho, acc.e[k].i, Z.e[k].r), mfma(rho, acc.e[k].r, Z.e[k].i)};
   return Z;
 }
 
-template <bool LAST, class TS, int NC, class TC, bool R12 = false>
-MAG_D void k_stout_bwd_body(const StoutBwdArgs<TS, NC>& a) {
-  int mu, sblk;
-  stencil_tile<sizeof(TC) == sizeof(double)>(a.g, mu, sblk);
-  const int s = sblk * BLOCK + threadIdx.x;
-  if (s >= a.g.V) return;
-  const Site p = site_of(a.g, s);
-  const M3<TC> Z = stout_six_terms<TS, NC, TC, R12>(a, p, mu);
+template <class TS, int NC, class TC, bool R12>
+MAG_D M3<TC> stout_six_terms(const StoutBwdArgs<TS, NC>& a, const Site& p, int mu) {
+  M3<TC> acc = zero3<TC>();
+  const int xpm = p.s + off_rt(a.g, p, mu, 1);
+#pragma unroll 1
+  for (int i = 0; i < 3; ++i) stout_plane<TS, NC, TC, R12>(a, p, mu, i + (i >= mu ? 1 : 0), xpm, acc);
+  return stout_Z<TS, NC, TC>(a, mu, p.s, acc);
+}
+
+// What follows Z at one link: the Lambda step of level k-1, or the force.
+template <bool LAST, class TS, int NC, class TC, bool R12>
+MAG_D void stout_bwd_link(const StoutBwdArgs<TS, NC>& a, int mu, int s, const M3<TC>& Z) {
   if (!LAST) {
     stout_lambda_link<TS, NC, TC, R12>(mu, s, Z, a.Ulo, a.Qlo, a.Clo, a.Lout, a.Wout);
   } else if (a.f.mag) {
@@ -761,10 +964,36 @@ MAG_D void k_stout_bwd_body(const StoutBwdArgs<TS, NC>& a) {
     force_epilogue<TS, NC, TC>(a.f, mu, s, Ux, f);
   }
 }
+
+template <bool LAST, class TS, int NC, class TC, bool R12 = false>
+MAG_D void k_stout_bwd_body(const StoutBwdArgs<TS, NC>& a) {
+  int mu, sblk;
+  stencil_tile<sizeof(TC) == sizeof(double)>(a.g, mu, sblk);
+  const int s = sblk * BLOCK + threadIdx.x;
+  if (s >= a.g.V) return;
+  const Site p = site_of(a.g, s);
+  const M3<TC> Z = stout_six_terms<TS, NC, TC, R12>(a, p, mu);
+  stout_bwd_link<LAST, TS, NC, TC, R12>(a, mu, s, Z);
+}
 template <bool LAST, class TS, int NC, class TC, bool R12 = false>
 __global__ __launch_bounds__(BLOCK) MAG_STENCIL_OCC void k_stout_bwd(StoutBwdArgs<TS, NC> a) { k_stout_bwd_body<LAST, TS, NC, TC, R12>(a); }
 template <bool LAST, class TS, int NC, class TC, bool R12 = false>
 __global__ __launch_bounds__(BLOCK) MAG_STENCIL_OCC void k_stout_bwd_b(const StoutBwdArgs<TS, NC>* t) { k_stout_bwd_body<LAST, TS, NC, TC, R12>(t[blockIdx.z]); }
+
+template <bool LAST, class TS, int NC, class TC, bool R12 = false>
+struct BwdStencil {
+  using Args = StoutBwdArgs<TS, NC>;
+  using Real = TC;
+  static constexpr int waves = stencil_waves<TC>();
+  MAG_D static M3<TC> share(const Args& a, const Site& p, int mu, int plane) {
+    M3<TC> acc = zero3<TC>();
+    stout_plane<TS, NC, TC, R12>(a, p, mu, plane + (plane >= mu ? 1 : 0), p.s + off_rt(a.g, p, mu, 1), acc);
+    return acc;
+  }
+  MAG_D static void finish(const Args& a, int mu, int s, const M3<TC>& acc) {
+    stout_bwd_link<LAST, TS, NC, TC, R12>(a, mu, s, stout_Z<TS, NC, TC>(a, mu, s, acc));
+  }
+};
 
 // Constrained runs with smearing: F from a stored Z_0 with the classes of
 // field-hmc.h:353-378: W = U Z (0), U(x+mu) Z(x+mu) - Z U (1, 10), 0 (100);

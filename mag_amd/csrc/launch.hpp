@@ -18,7 +18,7 @@ namespace mag {
 
 struct RecCall {
   const void* kb = nullptr;  // batched kernel entry, void(*)(const A*)
-  dim3 grid;
+  dim3 grid, block;
   size_t argsz = 0;
   std::vector<char> blob;  // argsz bytes per recorded chain
   void* table = nullptr;   // device copy of blob (set when the plan is built)
@@ -33,11 +33,12 @@ struct Recorder {
     chain = i;
     pos = 0;
   }
-  void add(const void* kb, dim3 grid, const void* args, size_t argsz) {
+  void add(const void* kb, dim3 grid, dim3 block, const void* args, size_t argsz) {
     if (chain == 0) {
       RecCall c;
       c.kb = kb;
       c.grid = grid;
+      c.block = block;
       c.argsz = argsz;
       calls.push_back(std::move(c));
     } else if (pos >= calls.size() || calls[pos].kb != kb || calls[pos].argsz != argsz ||
@@ -53,16 +54,41 @@ struct Recorder {
 };
 
 template <class A>
-int launch(mag_ctx c, const char* timer, void (*ks)(A), void (*kb)(const A*), dim3 grid, const A& a) {
+int launch(mag_ctx c, const char* timer, void (*ks)(A), void (*kb)(const A*), dim3 grid, const A& a,
+           int block = BLOCK) {
   if (c->rec) {
-    c->rec->add((const void*)kb, grid, &a, sizeof(A));
+    c->rec->add((const void*)kb, grid, dim3(block), &a, sizeof(A));
     return MAG_OK;
   }
   KTimer t(c, timer);
   A copy = a;
   void* args[] = {&copy};
-  HIPCHK(c, hipLaunchKernel((const void*)ks, grid, dim3(BLOCK), args, 0, c->stream));
+  HIPCHK(c, hipLaunchKernel((const void*)ks, grid, dim3(block), args, 0, c->stream));
   return MAG_OK;
+}
+
+// A stencil kernel in its split form: one wavefront per plane, 64 sites per block.
+template <class K>
+struct Stencil {};
+template <class A, class K>
+int launch_split(mag_ctx c, const char* timer, Stencil<K>, const Geom& g, const A& a) {
+  return launch(c, timer, k_split<K>, k_split_b<K>, grid_split(g), a, PLANE_THREADS);
+}
+// The split form up to SPLIT_MAX_SITES, else one thread per link (ks, kb). An
+// Iwasaki + 3-stout force, back to back, one thread per link -> split:
+//   FP32   4^4 88 -> 49 us, 8^4 92 -> 55, 10^4 102 -> 75, 12^4 120 -> 115, 14^4 176 -> 176, 16^4 257 -> 280
+//   FP64   4^4 119 -> 65,   8^4 135 -> 79, 10^4 147 -> 133, 12^4 232 -> 213, 14^4 371 -> 328
+// Below the line one thread per link leaves most SIMDs with one wavefront or
+// none; above it all are busy either way, and two of three wavefronts idle
+// while the first goes on costs 5-15 %. Six wavefronts (plane and side) took
+// 50 us at FP32 8^4 but 149 at 12^4; three groups of sites per block, every
+// wavefront going on with one, gave the split's gain back.
+constexpr int SPLIT_MAX_SITES = 1 << 15;
+template <class A, class K>
+int launch_stencil(mag_ctx c, const char* timer, void (*ks)(A), void (*kb)(const A*), Stencil<K> k, const Geom& g,
+                   const A& a) {
+  if (g.V <= SPLIT_MAX_SITES) return launch_split(c, timer, k, g, a);
+  return launch(c, timer, ks, kb, grid_stencil(g), a);
 }
 
 // Device-to-device copy of `bytes` (a multiple of 16) through a kernel.

@@ -16,9 +16,9 @@
 #endif
 
 // FP64 18-real links read as rows 0 and 1 with row 2 rebuilt, a bit per
-// kernel: 1 stout forward, 2 stout backward, 4 last backward, 8 link update
-// (on by default), 16 the top kernel at one wave per SIMD (off: as fast as
-// its full reads at two waves), 32 the thin-link force (off: within 1 %).
+// kernel: 1 stout forward, 2 stout backward, 4 last backward, 8 link update.
+// The rectangle staples of the top kernel and the thin-link force read whole
+// links (two rows: 2.16 -> 2.37 ms and 1.88 -> 2.13 ms at 32^4).
 #ifndef MAG_FP64_READ12
 #define MAG_FP64_READ12 15
 #endif
@@ -28,6 +28,15 @@ namespace mag {
 // whether Ops<TS, NC> reads its links as two rows in those kernels
 template <class TS, int NC>
 constexpr bool ops_read12(int bit) { return (MAG_FP64_READ12 & bit) != 0 && std::is_same<TS, double>::value && NC == 18; }
+
+// FP64 rectangle staples always take the split form. One thread per link
+// needs more than 256 VGPRs for them (it spills, or runs one wave per SIMD),
+// a plane's share fits; and three wavefronts on the same 64 sites ask L2 for
+// a third of the sites at a time. Thin force / top kernel, one thread per
+// link -> split: 12^4 59 -> 43 / 72 -> 57 us, 16^4 128 -> 110 / 161 -> 139,
+// 24^4 707 -> 569 / 857 -> 691, 32^4 2.17 -> 1.86 / 2.54 -> 2.15 ms.
+template <class TS>
+constexpr bool split_rectangles() { return std::is_same<TS, double>::value; }
 
 template <class TS, int NC>
 LinkView<TS, NC> lview(void* p, const Geom& g) { return LinkView<TS, NC>{(TS*)p, g.V}; }
@@ -41,6 +50,35 @@ int Ops<TS, NC>::link_update(mag_ctx c, const Geom& g, void* Uin, void* Uout, vo
   UpdateArgs<TS, NC> a{g, lview<TS, NC>(Uin, g), lview<TS, NC>(Uout, g), aview<TS>(P, g), eps, mag};
   constexpr bool R12 = ops_read12<TS, NC>(8);
   return launch(c, "link_update", k_link_update<TS, NC, TS, R12>, k_link_update_b<TS, NC, TS, R12>, grid_links(g), a);
+}
+
+// Thin-link force. Constrained runs: up to SPLIT_MAX_SITES the links with two
+// staple sums have blocks of their own, since with both sums in the stencil
+// every wavefront that meets such a link is twice as long (FP64 Iwasaki, mag
+// = 2: 4^4 58 -> 22 us, 8^4 61 -> 24, 12^4 107 -> 60; FP32 61 -> 17, 65 -> 18,
+// 64 -> 27). On larger lattices that costs little, and those blocks, which
+// share no neighbours with the stencil's in flight, cost more: 32^4 2.44 ms in
+// one thread per link, 2.86 with them.
+template <int ACT, class TS, int NC>
+int thin_force(mag_ctx c, ForceArgs<TS, NC> fa) {
+  const char* name = ACT == ACT_IWASAKI ? "force_iwasaki" : "force_wilson";
+  const Geom& g = fa.g;
+  if (fa.mag && g.V > SPLIT_MAX_SITES)
+    return launch(c, name, k_gauge_force<ACT, true, TS, NC, TS>, k_gauge_force_b<ACT, true, TS, NC, TS>,
+                  grid_stencil(g), fa);
+  if (fa.mag) {
+    int n = 0;
+    for (int mu = 0; mu < 4; ++mu) n = std::max(n, pair_count(g, mu, fa.mag));
+    fa.npair = (4 * ((n + 63) / 64) + 7) / 8 * 8;  // the stencil's blocks keep their XCDs
+    dim3 grid = grid_split(g);
+    grid.x += fa.npair;
+    return launch(c, name, k_cons_force<ACT, TS, NC, TS>, k_cons_force_b<ACT, TS, NC, TS>, grid, fa, PLANE_THREADS);
+  }
+  const Stencil<ForceStencil<ACT, false, TS, NC, TS>> split;
+  if constexpr (ACT == ACT_IWASAKI && split_rectangles<TS>()) return launch_split(c, name, split, g, fa);
+  else
+    return launch_stencil(c, name, k_gauge_force<ACT, false, TS, NC, TS>, k_gauge_force_b<ACT, false, TS, NC, TS>,
+                          split, g, fa);
 }
 
 // Force of the (possibly smeared) action on U with one of the epilogues
@@ -71,20 +109,7 @@ int Ops<TS, NC>::force(mag_ctx c, const Geom& g, void* U, const mag_action& act,
   fa.out = out;
   fa.eps = eps;
   const bool iw = act.type == MAG_IWASAKI;
-  if (act.n_stout <= 0) {
-    constexpr bool R12 = ops_read12<TS, NC>(32);
-    if (iw && act.mag)
-      return launch(c, "force_iwasaki", k_gauge_force<ACT_IWASAKI, true, TS, NC, TS, R12>,
-                    k_gauge_force_b<ACT_IWASAKI, true, TS, NC, TS, R12>, grid_stencil(g), fa);
-    if (iw)
-      return launch(c, "force_iwasaki", k_gauge_force<ACT_IWASAKI, false, TS, NC, TS, R12>,
-                    k_gauge_force_b<ACT_IWASAKI, false, TS, NC, TS, R12>, grid_stencil(g), fa);
-    if (act.mag)
-      return launch(c, "force_wilson", k_gauge_force<ACT_WILSON, true, TS, NC, TS, R12>,
-                    k_gauge_force_b<ACT_WILSON, true, TS, NC, TS, R12>, grid_stencil(g), fa);
-    return launch(c, "force_wilson", k_gauge_force<ACT_WILSON, false, TS, NC, TS, R12>,
-                  k_gauge_force_b<ACT_WILSON, false, TS, NC, TS, R12>, grid_stencil(g), fa);
-  }
+  if (act.n_stout <= 0) return iw ? thin_force<ACT_IWASAKI>(c, fa) : thin_force<ACT_WILSON>(c, fa);
   const int n = act.n_stout;
   constexpr bool R12 = ops_read12<TS, NC>(1), R12B = ops_read12<TS, NC>(2), R12L = ops_read12<TS, NC>(4);
   if ((r = ws->need_stout(n))) return r;
@@ -97,13 +122,13 @@ int Ops<TS, NC>::force(mag_ctx c, const Geom& g, void* U, const mag_action& act,
     if (NCN != NC && k == n - 1) {
       StoutFwdArgs<TS, NC, TS, NCN> fw{g, lview<TS, NC>(Ulev(k), g), aview<TS>(ws->Qs[k], g),
                                        mview<TS>(ws->Cs[k], g), lview<TS, NCN>(ws->Utop, g), act.rho, 1};
-      r = launch(c, "stout_fwd", k_stout_fwd<TS, NC, TS, NCN, TS>, k_stout_fwd_b<TS, NC, TS, NCN, TS>,
-                 grid_stencil(g), fw);
+      r = launch_stencil(c, "stout_fwd", k_stout_fwd<TS, NC, TS, NCN, TS>, k_stout_fwd_b<TS, NC, TS, NCN, TS>,
+                         Stencil<FwdStencil<TS, NC, TS, NCN, TS>>{}, g, fw);
     } else {
       StoutFwdArgs<TS, NC, TS, NC> fw{g, lview<TS, NC>(Ulev(k), g), aview<TS>(ws->Qs[k], g),
                                       mview<TS>(ws->Cs[k], g), lview<TS, NC>(ws->Us[k], g), act.rho, 1};
-      r = launch(c, "stout_fwd", k_stout_fwd<TS, NC, TS, NC, TS, R12>, k_stout_fwd_b<TS, NC, TS, NC, TS, R12>,
-                 grid_stencil(g), fw);
+      r = launch_stencil(c, "stout_fwd", k_stout_fwd<TS, NC, TS, NC, TS, R12>, k_stout_fwd_b<TS, NC, TS, NC, TS, R12>,
+                         Stencil<FwdStencil<TS, NC, TS, NC, TS, R12>>{}, g, fw);
     }
     if (r) return r;
   }
@@ -126,15 +151,17 @@ int Ops<TS, NC>::force(mag_ctx c, const Geom& g, void* U, const mag_action& act,
         r = launch(c, "stout_top", k_stout_top_tile<MAG_TOP_LDS>, k_stout_top_tile_b<MAG_TOP_LDS>, grid_stencil(g),
                    tp);
     }
-    // FP64 (both link formats: the top level U_n is stored as 18 reals)
-    constexpr bool R12T = (MAG_FP64_READ12 & 16) != 0 && std::is_same<TS, double>::value;
     if (!tiled) {
-      if (iw)
-        r = launch(c, "stout_top", k_stout_top<ACT_IWASAKI, TS, NC, TS, NCN, R12T>,
-                   k_stout_top_b<ACT_IWASAKI, TS, NC, TS, NCN, R12T>, grid_stencil(g), tp);
+      const Stencil<TopStencil<ACT_IWASAKI, TS, NC, TS, NCN>> split;
+      if (!iw)
+        r = launch_stencil(c, "stout_top", k_stout_top<ACT_WILSON, TS, NC, TS, NCN>,
+                           k_stout_top_b<ACT_WILSON, TS, NC, TS, NCN>,
+                           Stencil<TopStencil<ACT_WILSON, TS, NC, TS, NCN>>{}, g, tp);
+      else if constexpr (split_rectangles<TS>())
+        r = launch_split(c, "stout_top", split, g, tp);
       else
-        r = launch(c, "stout_top", k_stout_top<ACT_WILSON, TS, NC, TS, NCN>,
-                   k_stout_top_b<ACT_WILSON, TS, NC, TS, NCN>, grid_stencil(g), tp);
+        r = launch_stencil(c, "stout_top", k_stout_top<ACT_IWASAKI, TS, NC, TS, NCN>,
+                           k_stout_top_b<ACT_IWASAKI, TS, NC, TS, NCN>, split, g, tp);
     }
     if (r) return r;
   }
@@ -150,8 +177,8 @@ int Ops<TS, NC>::force(mag_ctx c, const Geom& g, void* U, const mag_action& act,
     bw.Lout = aview<TS>(ws->L[1 - cur], g);
     bw.Wout = mview<TS>(ws->W, g);
     bw.rho = act.rho;
-    if ((r = launch(c, "stout_bwd", k_stout_bwd<false, TS, NC, TS, R12B>, k_stout_bwd_b<false, TS, NC, TS, R12B>,
-                    grid_stencil(g), bw)))
+    if ((r = launch_stencil(c, "stout_bwd", k_stout_bwd<false, TS, NC, TS, R12B>,
+                            k_stout_bwd_b<false, TS, NC, TS, R12B>, Stencil<BwdStencil<false, TS, NC, TS, R12B>>{}, g, bw)))
       return r;
     cur = 1 - cur;
   }
@@ -166,8 +193,8 @@ int Ops<TS, NC>::force(mag_ctx c, const Geom& g, void* U, const mag_action& act,
     if ((r = ws->need_Z())) return r;
     bw.Zout = mview<TS>(ws->Z, g);
   }
-  if ((r = launch(c, "stout_bwd_force", k_stout_bwd<true, TS, NC, TS, R12L>, k_stout_bwd_b<true, TS, NC, TS, R12L>,
-                  grid_stencil(g), bw)))
+  if ((r = launch_stencil(c, "stout_bwd_force", k_stout_bwd<true, TS, NC, TS, R12L>,
+                          k_stout_bwd_b<true, TS, NC, TS, R12L>, Stencil<BwdStencil<true, TS, NC, TS, R12L>>{}, g, bw)))
     return r;
   if (!act.mag) return MAG_OK;
   // constrained: F from the stored Z_0 with the link classes
@@ -247,14 +274,14 @@ int Ops<TS, NC>::smeared_action_sums(mag_ctx c, const Geom& g, void* U, double r
     if (k == 0) {
       StoutFwdArgs<TS, NC, double, 18> fw{g, lview<TS, NC>(U, g), aview<double>(nullptr, g),
                                           mview<double>(nullptr, g), lview<double, 18>(dst, g), rho, 0};
-      r = launch(c, "stout_fwd_h", k_stout_fwd<TS, NC, double, 18, double>, k_stout_fwd_b<TS, NC, double, 18, double>,
-                 grid_stencil(g), fw);
+      r = launch_stencil(c, "stout_fwd_h", k_stout_fwd<TS, NC, double, 18, double>,
+                         k_stout_fwd_b<TS, NC, double, 18, double>, Stencil<FwdStencil<TS, NC, double, 18, double>>{}, g, fw);
     } else {
       StoutFwdArgs<double, 18, double, 18> fw{g, lview<double, 18>(wsd->Uh[(k - 1) & 1], g),
                                               aview<double>(nullptr, g), mview<double>(nullptr, g),
                                               lview<double, 18>(dst, g), rho, 0};
-      r = launch(c, "stout_fwd_h", k_stout_fwd<double, 18, double, 18, double>,
-                 k_stout_fwd_b<double, 18, double, 18, double>, grid_stencil(g), fw);
+      r = launch_stencil(c, "stout_fwd_h", k_stout_fwd<double, 18, double, 18, double>,
+                         k_stout_fwd_b<double, 18, double, 18, double>, Stencil<FwdStencil<double, 18, double, 18, double>>{}, g, fw);
     }
     if (r) return r;
   }
@@ -277,8 +304,8 @@ int Ops<TS, NC>::smear(mag_ctx c, const Geom& g, void* Uout, void* U, double rho
     if (dst == src) dst = (src == Uout) ? ws->Uaux : Uout;
     StoutFwdArgs<TS, NC, TS, NC> fw{g, lview<TS, NC>(src, g), aview<TS>(nullptr, g), mview<TS>(nullptr, g),
                                     lview<TS, NC>(dst, g), rho, 0};
-    if ((r = launch(c, "stout_fwd", k_stout_fwd<TS, NC, TS, NC, TS>, k_stout_fwd_b<TS, NC, TS, NC, TS>, grid_stencil(g),
-                    fw)))
+    if ((r = launch_stencil(c, "stout_fwd", k_stout_fwd<TS, NC, TS, NC, TS>, k_stout_fwd_b<TS, NC, TS, NC, TS>,
+                            Stencil<FwdStencil<TS, NC, TS, NC, TS>>{}, g, fw)))
       return r;
     src = dst;
   }

@@ -245,6 +245,9 @@ inline dim3 grid_links(const Geom& g) { return dim3((g.V + RT_BLOCK - 1) / RT_BL
 // 196 -> 179.
 inline dim3 grid_stencil(const Geom& g) { return dim3((4 * ((g.V + RT_BLOCK - 1) / RT_BLOCK) + 7) / 8 * 8, 1, 1); }
 
+// Stencils by planes (kernels.hpp): one block per group of 64 sites and direction, the groups dealt to 8 XCDs.
+inline dim3 grid_split(const Geom& g) { return dim3(8 * 4 * (((g.V + 63) / 64 + 7) / 8), 1, 1); }
+
 // ------------------------------------------------------------ workspace
 // Scratch of one lattice shape and storage format, owned by the context and
 // allocated on first use (never inside a timed trajectory once warm).

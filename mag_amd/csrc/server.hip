@@ -211,7 +211,7 @@ int build_batch(mag_server s, Batch* b) {
     HIPCHK(x, hipStreamBeginCapture(s->aux, hipStreamCaptureModeThreadLocal));
     for (auto& c : b->rec.calls) {
       void* args[] = {&c.table};
-      (void)hipLaunchKernel(c.kb, dim3(c.grid.x, c.grid.y, (unsigned)n), dim3(BLOCK), args, 0, s->aux);
+      (void)hipLaunchKernel(c.kb, dim3(c.grid.x, c.grid.y, (unsigned)n), c.block, args, 0, s->aux);
     }
     HIPCHK(x, hipStreamEndCapture(s->aux, &b->graph));
     HIPCHK(x, hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
@@ -246,7 +246,7 @@ int launch_batch(mag_server s, Batch* b) {
   } else {
     for (auto& c : b->rec.calls) {
       void* args[] = {&c.table};
-      HIPCHK(x, hipLaunchKernel(c.kb, dim3(c.grid.x, c.grid.y, (unsigned)n), dim3(BLOCK), args, 0, st));
+      HIPCHK(x, hipLaunchKernel(c.kb, dim3(c.grid.x, c.grid.y, (unsigned)n), c.block, args, 0, st));
     }
   }
   HIPCHK(x, hipMemcpyAsync(b->h_gather, b->gather, n * S_COUNT * sizeof(double), hipMemcpyDeviceToHost, st));
