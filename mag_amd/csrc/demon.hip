@@ -24,9 +24,6 @@ struct DemonTable {
   // dirs[mu][path][k]: 0..3 forward, 4..7 backward, -1 = end of path
   signed char dirs[4][NPATH][PLEN];
   unsigned char kind[NPATH];  // 0 plaquette, 1 rectangle, 2 chair, 3 twist
-  // paths [kbeg[k], kbeg[k+1]) are of kind k (the same for every direction),
-  // plaquettes of 3 links and the other kinds of 5
-  short kbeg[5];
 };
 
 // Paths of get_staple_dagger (field-hmc.h:226-240), get_rectangular_dagger
@@ -87,25 +84,6 @@ void build_table(DemonTable& t) {
         }
       }
   }
-  int k = 0;
-  for (int q = 0; q < NPATH; ++q)
-    while (k <= t.kind[q]) t.kbeg[k++] = (short)q;
-  while (k <= 4) t.kbeg[k++] = (short)NPATH;
-}
-
-// The checkerboard kernel's assumptions about the table: kinds in order,
-// plaquettes of 3 links, the rest of 5.
-bool table_ok(const DemonTable& t) {
-  for (int q = 0; q < NPATH; ++q) {
-    const int kd = t.kind[q];
-    if (q < t.kbeg[kd] || q >= t.kbeg[kd + 1]) return false;
-    for (int mu = 0; mu < 4; ++mu) {
-      int len = 0;
-      while (len < PLEN && t.dirs[mu][q][len] >= 0) ++len;
-      if (len != (kd == 0 ? 3 : 5)) return false;
-    }
-  }
-  return true;
 }
 
 struct DemonState {
@@ -267,14 +245,10 @@ __global__ __launch_bounds__(BLOCK) void k_staple_table_sum(LinkView<double, 18>
 // Every staple path of a link holds its MU-links at offsets with |d_nu| <= 2
 // and d_MU in {-1, 0, 1}, so two links of one class never meet in a path:
 // the updates of a class commute and each moves its own action change into
-// its own demons. Eight lanes per class member; hit counts in per-member slots.
-// The lanes sum one kind of path at a time (one accumulator; the finished
-// sums wait in LDS), each lane the same paths in the same order as a single
-// loop over all paths, so the sums are bitwise those of that loop.
+// its own demons. Hit counts in per-member slots.
 struct DemonClassArgs {
   LinkView<double, 18> U;
   Geom g;
-  const DemonTable* tab;
   double* E[4];   // per-link demon energies, [mu][site] each
   double* cnt;    // [thread][2]: accept, reject
   double emax;
@@ -283,173 +257,254 @@ struct DemonClassArgs {
   int nthr;           // class members
 };
 
-// LPL lanes per class member, 64 / LPL members per wavefront: lane sub of a
-// member sums paths sub, sub + LPL, ..., a butterfly over its LPL lanes
-// (fixed order) reduces the four 3x3 sums, and its lane 0 makes the hits.
-// Members are enumerated x0 fastest, so the lanes of one sub-index read
-// neighbouring sites. Surplus lanes of the last wavefront repeat the last
-// member and write nothing. Sweep of a 32^4 lattice on MI355X: 387 ms with
-// 64 lanes per member (every lane's gather its own cache lines), 155 ms with
-// 16, 142 ms with 8, 193 ms with 4 (too few wavefronts per class). A class
-// launch at 32^4 is 1,024 one-wave blocks, one wave per SIMD, so the path
-// loads are latency-bound: requesting a path's links together before its
-// products (one round trip per path, not one per link) took the sweep from
-// 107 to 79 ms; 16 lanes at 2 waves per SIMD gave 77.5 ms, and requesting
-// the next path's links during this path's products 93 ms (AGPR copies).
-constexpr int DEMON_LPL = 8;
+// The staple sums of a member, by signed transverse directions n and l on
+// different axes (24 pairs). Writing a path as the directions it steps along,
+// with m for +MU:
+//   twist   n m l -n -l,  n l m -n -l,  n l -n m -l              every (n, l)
+//   chair   n m l l n,    n l m l n,    n l l m n                signs of n, l differ
+//           n l m -l -n,  and n m l -l -n, n l -l m -n           signs alike
+// (the table's defects kept). The last two step back along a link at once and
+// are the plaquette staple n m -n: each staple four times in all. The others
+// share factors: with A1 = U_m(x+n) U_l(x+n+m), A2 = U_l(x+n) U_m(x+n+l), both
+// from x+n to x+n+l+m, each pair gives
+//   twist   U_n [(A1 + A2) U_-n + U_l U_-n U_m] U_-l
+//   chair   U_n [(A1 + A2) U_l + U_l U_l U_m] U_n      or      U_n A2 U_-l U_-n
+// 13-16 links and about 10 products against 30 links and 24 products path by
+// path. The 24 plaquette and rectangle staples go one to each pair.
+//
+// A block is ten members by four wavefronts, one per choice of signs, so that
+// the form and every dagger are the same across a wavefront; a lane is one of
+// its six axis pairs of one member, ten neighbouring members side by side.
+// The shares are summed in LDS in a fixed order, one kind of sum at a time;
+// then four lanes per member, one per kind, make the two hits. What bounds a
+// class launch on lattices up to 16^4 (52 blocks) is the latency of one
+// wavefront, above that one wavefront per SIMD (460 registers: a lane asks
+// for all its links at once; held to two, it spills 856 bytes and takes 1.5
+// to 1.9 times as long). Launch of a class: 4^4 77 -> 14 us, 16^4 78 -> 18,
+// 24^4 90 -> 43, 32^4 152 -> 103, against eight lanes per member that walked
+// the 168 paths one by one.
+constexpr int DEMON_MEMBERS = 10, DEMON_PAIRS = 6;
 // MAG_DEMON_READ12 = 1: the path links are read as rows 0 and 1 with row 2
-// rebuilt (the gathers bound the class kernel; the links stay in SU(3)).
+// rebuilt (the links stay in SU(3)).
 #ifndef MAG_DEMON_READ12
 #define MAG_DEMON_READ12 1
 #endif
-// The paths of one kind, of LEN links each, that lane sub of a member sums
-// (q = sub mod LPL, in increasing q, as one loop over all paths would give
-// it): the links of a path are all requested before its products (sdir is
-// the direction's path table in LDS).
-template <int LPL, int LEN>
-MAG_D void demon_kind_sum(const DemonClassArgs& A, const signed char* sdir, int qa, int qb, int sub, const int x[4],
-                          M3<double>& X) {
-  X = zero3<double>();
-#pragma unroll 1
-  for (int q = qa + ((sub - qa) % LPL + LPL) % LPL; q < qb; q += LPL) {
-    int y[4] = {x[0], x[1], x[2], x[3]};
-    M3<double> l[LEN];
-    bool back[LEN];
+
+struct DemonPos {
+  int x[4], s;
+};
+// The link of a step along axis k, forward or backward, from y, which moves on.
+template <bool BACK>
+MAG_D M3<double> demon_step(const DemonClassArgs& A, DemonPos& y, int k) {
+  const int s0 = y.s;
 #pragma unroll
-    for (int j = 0; j < LEN; ++j) {
-      const int d = sdir[q * PLEN + j];
-      const int k = d & 3;
-      back[j] = d >= 4;
-      if (back[j]) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (i == k) y[i] = (y[i] == 0) ? A.g.L[i] - 1 : y[i] - 1;
-      }
-      const int sy = y[0] + A.g.S[1] * y[1] + A.g.S[2] * y[2] + A.g.S[3] * y[3];
-      l[j] = MAG_DEMON_READ12 ? A.U.template load_r2<double>(k, sy) : A.U.template load<double>(k, sy);
-      if (!back[j]) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (i == k) y[i] = (y[i] == A.g.L[i] - 1) ? 0 : y[i] + 1;
-      }
+  for (int i = 0; i < 4; ++i)
+    if (i == k) {
+      const int v = y.x[i], L = A.g.L[i];
+      const int w = BACK ? (v == 0 ? L - 1 : v - 1) : (v == L - 1 ? 0 : v + 1);
+      y.x[i] = w;
+      y.s += (w - v) * A.g.S[i];
     }
-    __builtin_amdgcn_sched_barrier(0);  // keep the path's loads ahead of its products
-    M3<double> m;
-#pragma unroll
-    for (int j = 0; j < LEN; ++j) {
-      if (MAG_DEMON_READ12) reconstruct_row2(l[j]);
-      if (j == 0) m = back[0] ? dag(l[0]) : l[0];
-      else m = back[j] ? mul_nd(m, l[j]) : mul(m, l[j]);
-    }
-    add_to(X, m);
-  }
-  // butterfly over the member's lanes: each ends with the full sum
-#pragma unroll
-  for (int off = LPL / 2; off >= 1; off >>= 1)
-#pragma unroll
-    for (int e = 0; e < 9; ++e) {
-      X.e[e].r += __shfl_xor(X.e[e].r, off, 64);
-      X.e[e].i += __shfl_xor(X.e[e].i, off, 64);
-    }
+  const M3<double> m = A.U.template load_su3<double, MAG_DEMON_READ12 != 0>(k, BACK ? y.s : s0);
+  return BACK ? dag(m) : m;
+}
+MAG_D M3<double> mul_su3(const M3<double>& a, const M3<double>& b) {
+  M3<double> c = mul_r2(a, b);
+  reconstruct_row2(c);
+  return c;
 }
 
-template <int MU, int LPL>
-__global__ __launch_bounds__(64) void k_demon_class(DemonClassArgs A) {
-  constexpr int MPW = 64 / LPL;
-  __shared__ signed char sdir[NPATH * PLEN];
-  __shared__ double sum[MPW][4][18];  // a member's four staple sums, written by its lane 0
-  const int lane = threadIdx.x;
-  for (int i = lane; i < NPATH * PLEN; i += 64) sdir[i] = (&A.tab->dirs[MU][0][0])[i];
-  __syncthreads();
-  const int sub = lane % LPL, mem = lane / LPL;
-  const int t0 = blockIdx.x * MPW + mem;
-  const bool live = t0 < A.nthr;
-  const int t = live ? t0 : A.nthr - 1;
-  int x[4], r = t, c = A.cls;
+// One lane's shares: twist, chair (without the plaquette staples) and one
+// plaquette or rectangle staple; SN, SL: whether n, l point backward. j = 0 or
+// 1 numbers the axis of l; with SL forward j = 0 holds the plaquette staple.
+template <int MU, bool SN, bool SL>
+MAG_D void demon_shares(const DemonClassArgs& A, const DemonPos& x, int n, int l, int j, M3<double>& tw,
+                        M3<double>& ch, M3<double>& pr) {
+  DemonPos yn = x;
+  const M3<double> Un = demon_step<SN>(A, yn, n);  // x -> x+n
+  DemonPos ym = yn, yl = yn;
+  const M3<double> m1 = demon_step<false>(A, ym, MU);  // x+n -> x+n+m
+  const M3<double> l1 = demon_step<SL>(A, yl, l);      // x+n -> x+n+l
+  DemonPos ye = ym, t = yl;
+  const M3<double> l2 = demon_step<SL>(A, ye, l);      // x+n+m -> x+n+l+m
+  const M3<double> m2 = demon_step<false>(A, t, MU);   // x+n+l -> x+n+l+m
+  const M3<double> A2 = mul_su3(l1, m2);
+  const M3<double> S = add(mul_su3(m1, l2), A2);
+  {
+    t = ye;
+    M3<double> B = mul(S, demon_step<!SN>(A, t, n));   // -> x+l+m
+    DemonPos u = yl;
+    M3<double> C = mul_r2(l1, demon_step<!SN>(A, u, n));  // -> x+l
+    add_to(B, mul_su3(C, demon_step<false>(A, u, MU)));   // -> x+l+m
+    tw = mul(Un, mul(B, demon_step<!SL>(A, t, l)));       // -> x+m
+  }
+  t = ye;
+  if (SN != SL) {
+    M3<double> B = mul(S, demon_step<SL>(A, t, l));       // -> x+n+2l+m
+    DemonPos u = yl;
+    M3<double> C = mul_r2(l1, demon_step<SL>(A, u, l));   // -> x+n+2l
+    add_to(B, mul_su3(C, demon_step<false>(A, u, MU)));   // -> x+n+2l+m
+    ch = mul(Un, mul(B, demon_step<SN>(A, t, n)));        // -> x+2n+2l+m
+  } else {
+    M3<double> B = mul_r2(mul_r2(Un, A2), demon_step<!SL>(A, t, l));  // -> x+n+m
+    ch = mul_su3(B, demon_step<!SN>(A, t, n));                        // -> x+m
+  }
+  if (!SL) {
+    t = ym;
+    M3<double> B = mul_r2(Un, m1);
+    if (j == 0) {  // n m -n
+      pr = mul_su3(B, demon_step<!SN>(A, t, n));
+    } else {  // n m m -n -m
+      B = mul_r2(B, demon_step<false>(A, t, MU));
+      B = mul_r2(B, demon_step<!SN>(A, t, n));
+      pr = mul_su3(B, demon_step<true>(A, t, MU));
+    }
+  } else if (j == 0) {  // n n m -n -n
+    t = yn;
+    M3<double> B = mul_r2(Un, demon_step<SN>(A, t, n));
+    B = mul_r2(B, demon_step<false>(A, t, MU));
+    B = mul_r2(B, demon_step<!SN>(A, t, n));
+    pr = mul_su3(B, demon_step<!SN>(A, t, n));
+  } else {  // -m n m m -n
+    t = x;
+    M3<double> B = demon_step<true>(A, t, MU);
+    B = mul_r2(B, demon_step<SN>(A, t, n));
+    B = mul_r2(B, demon_step<false>(A, t, MU));
+    B = mul_r2(B, m1);
+    t = ym;
+    pr = mul_su3(B, demon_step<!SN>(A, t, n));
+  }
+}
+
+// Proposal of hit n of link (x, mu): random_su3_from_su2(0.9) (field-matrix.h:36-65).
+MAG_D M3<double> demon_proposal(const DemonClassArgs& A, uint32_t link, int n) {
+  const u32x4 w0 = rng_draw(A.seed, RNG_DEMON, (uint64_t)A.sweep, link, 3 * n);
+  const u32x4 w1 = rng_draw(A.seed, RNG_DEMON, (uint64_t)A.sweep, link, 3 * n + 1);
+  const u32x4 w2 = rng_draw(A.seed, RNG_DEMON, (uint64_t)A.sweep, link, 3 * n + 2);
+  const double a0 = 0.9 + (1. - 0.9) * rng_u01(w0.x, w0.y);
+  double a1 = -1. + 2. * rng_u01(w0.z, w0.w);
+  double a2 = -1. + 2. * rng_u01(w1.x, w1.y);
+  double a3 = -1. + 2. * rng_u01(w1.z, w1.w);
+  const double nrm = sqrt((1. - a0 * a0) / (a1 * a1 + a2 * a2 + a3 * a3));
+  a1 *= nrm;
+  a2 *= nrm;
+  a3 *= nrm;
+  M3<double> m = unit3<double>();
+  switch (w2.x % 3) {
+    case 0: m(1, 1) = {a0, a3}; m(1, 2) = {a2, a1}; m(2, 1) = {-a2, a1}; m(2, 2) = {a0, -a3}; break;
+    case 1: m(0, 0) = {a0, a3}; m(0, 2) = {a2, a1}; m(2, 0) = {-a2, a1}; m(2, 2) = {a0, -a3}; break;
+    default: m(0, 0) = {a0, a3}; m(0, 1) = {a2, a1}; m(1, 0) = {-a2, a1}; m(1, 1) = {a0, -a3}; break;
+  }
+  return m;
+}
+
+// Member t of a class of direction MU.
+template <int MU>
+MAG_D DemonPos demon_member(const DemonClassArgs& A, int t) {
+  DemonPos p;
+  p.s = 0;
+  int c = A.cls;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int step = (i == MU) ? 2 : 4;
-    const int h = r % (A.g.L[i] / step);
-    r /= A.g.L[i] / step;
+    const int step = (i == MU) ? 2 : 4, n = A.g.L[i] / step, h = t % n;
+    t /= n;
     if (i == MU) {
-      x[i] = 2 * h + A.a;
+      p.x[i] = 2 * h + A.a;
     } else {
-      x[i] = 4 * h + (c & 3);
+      p.x[i] = 4 * h + (c & 3);
       c >>= 2;
     }
+    p.s += p.x[i] * A.g.S[i];
   }
-  const int s = x[0] + A.g.S[1] * x[1] + A.g.S[2] * x[2] + A.g.S[3] * x[3];
-  // the four staple sums (same paths and kinds as the sequential demon), one
-  // kind at a time
-#pragma unroll 1
-  for (int kd = 0; kd < 4; ++kd) {
-    M3<double> X;
-    if (kd == 0) demon_kind_sum<LPL, 3>(A, sdir, A.tab->kbeg[0], A.tab->kbeg[1], sub, x, X);
-    else demon_kind_sum<LPL, 5>(A, sdir, A.tab->kbeg[kd], A.tab->kbeg[kd + 1], sub, x, X);
-    if (sub == 0) {
-#pragma unroll
-      for (int e = 0; e < 9; ++e) {
-        sum[mem][kd][2 * e] = X.e[e].r;
-        sum[mem][kd][2 * e + 1] = X.e[e].i;
-      }
-    }
-  }
-  if (sub != 0 || !live) return;
-  M3<double> X[4];
+  return p;
+}
+
+template <int MU>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void k_demon_class(DemonClassArgs A) {
+  constexpr int NM = DEMON_MEMBERS, NP = DEMON_PAIRS;
+  __shared__ double buf[4][NP][NM][18];  // one kind of share at a time
+  __shared__ double tot[4][NM][18];      // plaquette, rectangle, chair, twist sums
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  // lanes 60-63 repeat the last pair and write nothing, members past the end the last member
+  const int pair = min(lane / NM, NP - 1), mem = lane % NM;
+  const DemonPos x = demon_member<MU>(A, min((int)blockIdx.x * NM + mem, A.nthr - 1));
+  const int i = pair >> 1, j = pair & 1;
+  const int n = i + (i >= MU ? 1 : 0);  // axis of n; that of l is the j-th of the other two
+  int l = 0, seen = 0;
 #pragma unroll
   for (int k = 0; k < 4; ++k)
+    if (k != MU && k != n && seen++ == j) l = k;
+  M3<double> sh[3];
+  switch (wave) {
+    case 0: demon_shares<MU, false, false>(A, x, n, l, j, sh[0], sh[1], sh[2]); break;
+    case 1: demon_shares<MU, false, true>(A, x, n, l, j, sh[0], sh[1], sh[2]); break;
+    case 2: demon_shares<MU, true, false>(A, x, n, l, j, sh[0], sh[1], sh[2]); break;
+    default: demon_shares<MU, true, true>(A, x, n, l, j, sh[0], sh[1], sh[2]); break;
+  }
+  const int e = threadIdx.x % 18, m = threadIdx.x / 18;  // the element that a thread sums
 #pragma unroll
-    for (int e = 0; e < 9; ++e) X[k].e[e] = {sum[mem][k][2 * e], sum[mem][k][2 * e + 1]};
-  // plaquette and rectangle sums are used daggered, chair and twist as they are
-  X[0] = dag(X[0]);
-  X[1] = dag(X[1]);
-  double E[4];
+  for (int r = 0; r < 3; ++r) {
+    if (lane < NP * NM) {
 #pragma unroll
-  for (int k = 0; k < 4; ++k) E[k] = __builtin_nontemporal_load(&A.E[k][(size_t)MU * A.g.V + s]);
-  M3<double> v = A.U.template load_nt<double>(MU, s);
+      for (int k = 0; k < 9; ++k) {
+        buf[wave][pair][mem][2 * k] = sh[r].e[k].r;
+        buf[wave][pair][mem][2 * k + 1] = sh[r].e[k].i;
+      }
+    }
+    __syncthreads();
+    if (m < NM) {
+      double a = 0., b = 0.;
+      for (int w = 0; w < 4; ++w)
+        for (int q = 0; q < NP; ++q) {
+          const double v = buf[w][q][m][e];
+          if (r == 2 && (w & 1) == 0 && (q & 1) == 0) b += v;  // plaquette staples
+          else a += v;
+        }
+      if (r == 0) tot[3][m][e] = a;
+      if (r == 1) tot[2][m][e] = a;
+      if (r == 2) {
+        tot[1][m][e] = a;
+        tot[0][m][e] = b;
+        tot[2][m][e] += 4. * b;
+      }
+    }
+    __syncthreads();
+  }
+  // the hits: lane 4 m + k holds kind k of member m
+  if (wave != 3 || lane >= 4 * NM) return;
+  const int hm = lane >> 2, k = lane & 3, t = (int)blockIdx.x * NM + hm;
+  if (t >= A.nthr) return;
+  const int s = demon_member<MU>(A, t).s;
   const uint32_t link = (uint32_t)s * 4u + (uint32_t)MU;
+  M3<double> X;
+#pragma unroll
+  for (int q = 0; q < 9; ++q) X.e[q] = {tot[k][hm][2 * q], tot[k][hm][2 * q + 1]};
+  // plaquette and rectangle sums are used daggered, chair and twist as they are
+  if (k < 2) X = dag(X);
+  M3<double> v = A.U.template load<double>(MU, s);
+  double E = A.E[k][(size_t)MU * A.g.V + s];
   double acc = 0., rej = 0.;
+  double old = retrace_mul(v, X);
 #pragma unroll 1
-  for (int n = 0; n < 2; ++n) {
-    const u32x4 w0 = rng_draw(A.seed, RNG_DEMON, (uint64_t)A.sweep, link, 3 * n);
-    const u32x4 w1 = rng_draw(A.seed, RNG_DEMON, (uint64_t)A.sweep, link, 3 * n + 1);
-    const u32x4 w2 = rng_draw(A.seed, RNG_DEMON, (uint64_t)A.sweep, link, 3 * n + 2);
-    const double a0 = 0.9 + (1. - 0.9) * rng_u01(w0.x, w0.y);
-    double a1 = -1. + 2. * rng_u01(w0.z, w0.w);
-    double a2 = -1. + 2. * rng_u01(w1.x, w1.y);
-    double a3 = -1. + 2. * rng_u01(w1.z, w1.w);
-    const double nrm = sqrt((1. - a0 * a0) / (a1 * a1 + a2 * a2 + a3 * a3));
-    a1 *= nrm;
-    a2 *= nrm;
-    a3 *= nrm;
-    M3<double> m = unit3<double>();
-    switch (w2.x % 3) {
-      case 0: m(1, 1) = {a0, a3}; m(1, 2) = {a2, a1}; m(2, 1) = {-a2, a1}; m(2, 2) = {a0, -a3}; break;
-      case 1: m(0, 0) = {a0, a3}; m(0, 2) = {a2, a1}; m(2, 0) = {-a2, a1}; m(2, 2) = {a0, -a3}; break;
-      default: m(0, 0) = {a0, a3}; m(0, 1) = {a2, a1}; m(1, 0) = {-a2, a1}; m(1, 1) = {a0, -a3}; break;
-    }
-    const M3<double> mv = mul(m, v);
-    double dS[4];
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      dS[k] = -retrace_mul(mv, X[k]) + retrace_mul(v, X[k]);
-      ok = ok && (E[k] - dS[k] > -A.emax) && (E[k] - dS[k] < A.emax);
-    }
-    if (ok) {
+  for (int h = 0; h < 2; ++h) {
+    const M3<double> mv = mul(demon_proposal(A, link, h), v);
+    const double now = retrace_mul(mv, X), dS = old - now;
+    const bool ok = (E - dS > -A.emax) && (E - dS < A.emax);
+    if (((__ballot(ok) >> (lane & ~3)) & 15) == 15) {
       v = mv;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) E[k] -= dS[k];
+      old = now;
+      E -= dS;
       acc += 1.;
     } else {
       rej += 1.;
     }
   }
-  A.U.store_nt(MU, s, v);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) __builtin_nontemporal_store(E[k], &A.E[k][(size_t)MU * A.g.V + s]);
-  A.cnt[(size_t)t * 2] += acc;
-  A.cnt[(size_t)t * 2 + 1] += rej;
+  A.E[k][(size_t)MU * A.g.V + s] = E;
+  if (k == 0) {
+    A.U.template store<double>(MU, s, v);
+    A.cnt[(size_t)t * 2] += acc;
+    A.cnt[(size_t)t * 2 + 1] += rej;
+  }
 }
 
 }  // namespace
@@ -513,29 +568,16 @@ extern "C" int mag_demon_checkerboard(mag_field U, mag_field Ep, mag_field Er, m
   if ((r = ws->need_cnt())) return r;  // V doubles >= 2 per thread
   double* cnt = (double*)ws->Cnt;
   if ((r = fill_dev(c, cnt, 0., 2 * nthr))) return r;
-  DemonTable* ht = new DemonTable();
-  build_table(*ht);
-  if (!table_ok(*ht)) {
-    delete ht;
-    return fail(c, MAG_ERR_STATE, "demon path table does not have the layout the class kernel assumes");
-  }
-  DemonTable* dt = nullptr;
-  r = dev_alloc(c, (void**)&dt, sizeof(DemonTable));
-  if (!r && hipMemcpyAsync(dt, ht, sizeof(DemonTable), hipMemcpyHostToDevice, c->stream) != hipSuccess)
-    r = fail(c, MAG_ERR_DEVICE, "demon table upload failed");
   DemonClassArgs A{};
   A.U = LinkView<double, 18>{(double*)U->p, U->g.V};
   A.g = U->g;
-  A.tab = dt;
   for (int k = 0; k < 4; ++k) A.E[k] = (double*)Ef[k]->p;
   A.cnt = cnt;
   A.emax = E_max;
   A.seed = seed;
-  constexpr int LPL = DEMON_LPL, MPW = 64 / LPL;
-  void (*ks[4])(DemonClassArgs) = {k_demon_class<0, LPL>, k_demon_class<1, LPL>, k_demon_class<2, LPL>,
-                                   k_demon_class<3, LPL>};
+  void (*ks[4])(DemonClassArgs) = {k_demon_class<0>, k_demon_class<1>, k_demon_class<2>, k_demon_class<3>};
   A.nthr = nthr;
-  const dim3 grid((nthr + MPW - 1) / MPW);
+  const dim3 grid((nthr + DEMON_MEMBERS - 1) / DEMON_MEMBERS);
   for (int sw = 0; sw < nsweeps && !r; ++sw) {
     A.sweep = sw;
     for (int mu = 0; mu < 4 && !r; ++mu)
@@ -543,7 +585,7 @@ extern "C" int mag_demon_checkerboard(mag_field U, mag_field Ep, mag_field Er, m
         A.a = cl & 1;
         A.cls = cl >> 1;
         KTimer t(c, "demon_checkerboard");
-        hipLaunchKernelGGL(ks[mu], grid, dim3(64), 0, c->stream, A);
+        hipLaunchKernelGGL(ks[mu], grid, dim3(256), 0, c->stream, A);
         if (hipGetLastError() != hipSuccess) r = fail(c, MAG_ERR_DEVICE, "demon launch failed");
       }
   }
@@ -552,9 +594,6 @@ extern "C" int mag_demon_checkerboard(mag_field U, mag_field Ep, mag_field Er, m
                  hipSuccess ||
              hipStreamSynchronize(c->stream) != hipSuccess))
     r = fail(c, MAG_ERR_DEVICE, "demon download failed");
-  (void)hipStreamSynchronize(c->stream);
-  dev_free(c, dt, dt ? sizeof(DemonTable) : 0);
-  delete ht;
   if (r) return r;
   if (acc_rej) {
     double a = 0., b = 0.;
