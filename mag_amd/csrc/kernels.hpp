@@ -1291,42 +1291,108 @@ __global__ __launch_bounds__(BLOCK) void k_reunitarize_b(const ReunitArgs<TS, NC
 }
 
 // Wilson loops (field-wloop.h:26-98): Re Tr of the R x T loop for every
-// permutation of r, per site, FP64.
+// permutation of r, per site, FP64. A loop is Tr[P(x) T(x+r) (T(x) P(x+T))^+]
+// with P the spatial and T the temporal line, both followed forward only. Two
+// wavefronts share a site's loop: one multiplies P(x) T(x+r), the other goes
+// on from T(x), formed once per site, with P(x+T) and hands its product over
+// in LDS. Half the serial chain each, and a product and two links fit 256
+// registers (168 on FP32 links), two (three) wavefronts per SIMD; one thread
+// per loop pays for every load of 2 (R + T) links in turn. R = T = 4, per call:
+// 8^4 23 -> 9 us, 24^3 x 32 312 -> 152, 32^4 609 -> 390; R = T = 1 100 -> 65
+// and 204 -> 175; FP32 links 24^3 x 32 140 -> 117 (R = T = 1 41 -> 43).
 struct WloopArgs {
   Geom g;
-  int nperm;
+  int nperm, per;  // permutations, of them per grid row
   int r[6][3];
   int T;
 };
+constexpr int WLOOP_SITES = BLOCK / 2;
+// Block of WLOOP_SITES sites that block b of nb takes: XCD k (b mod 8) has a
+// contiguous run of a walk with x3 fastest where an x3 slice is whole blocks
+// (the temporal lines of the sites that share them then meet in its L2: 24^3 x
+// 32, R = T = 4, 185 -> 151 us), else in site order.
+MAG_HD int wloop_block(const Geom& g, int b, int nb) {
+  const int k = b % 8, r = nb % 8;
+  const int t = k * (nb / 8) + (k < r ? k : r) + b / 8;
+  return g.S[3] % WLOOP_SITES == 0 ? (t % g.L[3]) * (g.S[3] / WLOOP_SITES) + t / g.L[3] : t;
+}
+
+MAG_D void site_step(const Geom& g, Site& y, int d) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (i == d) {
+      const int v = y.x[i], w = v + 1 == g.L[i] ? 0 : v + 1;
+      y.x[i] = w;
+      y.s += (w - v) * g.S[i];
+    }
+}
+// m times the n links along direction d from y on, each requested one step
+// ahead; y moves to the end. FRESH: m = their product.
+template <bool FRESH, class TS, int NC>
+MAG_D void line_right(const LinkView<TS, NC>& U, const Geom& g, Site& y, int d, int n, M3<double>& m) {
+  if (n <= 0) return;
+  auto l = U.raw(d, y.s);
+  int k = 1;
+  if (FRESH) {
+    site_step(g, y, d);
+    m = l.template mat<double>();
+    if (n == 1) return;
+    l = U.raw(d, y.s);
+    k = 2;
+  }
+#pragma unroll 1
+  for (; k < n; ++k) {
+    site_step(g, y, d);
+    const auto nx = U.raw(d, y.s);
+    m = mul(m, l.template mat<double>());
+    l = nx;
+  }
+  site_step(g, y, d);
+  m = mul(m, l.template mat<double>());
+}
 template <class TS, int NC>
-__global__ __launch_bounds__(BLOCK) void k_wilson_loop(LinkView<TS, NC> U, WloopArgs a, double* part) {
-  const int s = blockIdx.x * BLOCK + threadIdx.x;
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(TS) == 4 ? 3 : 2))) void k_wilson_loop(
+    LinkView<TS, NC> U, WloopArgs a, double* part) {
+  __shared__ double hand[2][18][WLOOP_SITES];
+  const int blk = wloop_block(a.g, blockIdx.x, gridDim.x), t = threadIdx.x & (WLOOP_SITES - 1);
+  const bool second = __builtin_amdgcn_readfirstlane((int)threadIdx.x / WLOOP_SITES) != 0;
+  const int s = blk * WLOOP_SITES + t;
+  const Site x = site_of(a.g, min(s, a.g.V - 1));
+  Site xt = x;
+  M3<double> time = unit3<double>();
+  if (second) line_right<true>(U, a.g, xt, 3, a.T, time);  // T(x)
   double acc = 0.;
-  if (s < a.g.V) {
-    for (int q = 0; q < a.nperm; ++q) {
-      Site y = site_of(a.g, s);
-      M3<double> m = unit3<double>();
-      auto fwd = [&](int d) {
-        m = mul(m, U.template load<double>(d, y.s));
-        y.s += off_rt(a.g, y, d, 1);
-        y.x[d] = (y.x[d] + 1 == a.g.L[d]) ? 0 : y.x[d] + 1;
-      };
-      auto bwd = [&](int d) {
-        y.s += off_rt(a.g, y, d, -1);
-        y.x[d] = (y.x[d] == 0) ? a.g.L[d] - 1 : y.x[d] - 1;
-        m = mul_nd(m, U.template load<double>(d, y.s));
-      };
-      for (int i = 0; i < 3; ++i)
-        for (int j = 0; j < a.r[q][i]; ++j) fwd(i);
-      for (int j = 0; j < a.T; ++j) fwd(3);
-      for (int i = 2; i >= 0; --i)
-        for (int j = 0; j < a.r[q][i]; ++j) bwd(i);
-      for (int j = 0; j < a.T; ++j) bwd(3);
-      acc += retrace(m);
+  const int q1 = min(a.nperm, (int)(blockIdx.y + 1) * a.per);
+#pragma unroll 1
+  for (int q = blockIdx.y * a.per; q < q1; ++q) {
+    Site y = second ? xt : x;
+    M3<double> m = time;
+    int i = 0;
+    if (!second) {  // the first line is its own product (the last one, T, when r is zero)
+      while (i < 3 && a.r[q][i] <= 0) ++i;
+      line_right<true>(U, a.g, y, i, i < 3 ? a.r[q][i] : a.T, m);
+      ++i;
+    }
+#pragma unroll 1
+    for (; i < (second ? 3 : 4); ++i) line_right<false>(U, a.g, y, i, i < 3 ? a.r[q][i] : a.T, m);
+    double(*h)[WLOOP_SITES] = hand[q & 1];  // the other half is read meanwhile
+    if (second) {
+#pragma unroll
+      for (int k = 0; k < 9; ++k) {
+        h[2 * k][t] = m.e[k].r;
+        h[2 * k + 1][t] = m.e[k].i;
+      }
+    }
+    __syncthreads();
+    if (!second) {
+      M3<double> w;
+#pragma unroll
+      for (int k = 0; k < 9; ++k) w.e[k] = {h[2 * k][t], h[2 * k + 1][t]};
+      acc += retrace_mul_nd(m, w);
     }
   }
-  const double t = block_sum(acc);
-  if (threadIdx.x == 0) part[blockIdx.x] = t;
+  const double sum = block_sum(s < a.g.V ? acc : 0.);
+  if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blk] = sum;
 }
 
 // Final reduction of block partials, one block, fixed order: each thread

@@ -183,16 +183,26 @@ struct LinkView {
   TS* p;
   int V;
   using PK = Packed<TS, NC>;
-  template <class TC, bool NT>
-  MAG_D M3<TC> get(int mu, int s) const {
+  // A link as stored (to be held while it is on its way) and as a matrix.
+  struct Raw {
     TS r[NC];
-    PK::template get<NC, NT>(p, V, mu, s, r);
-    M3<TC> m;
+    template <class TC>
+    MAG_D M3<TC> mat() const {
+      M3<TC> m;
 #pragma unroll
-    for (int k = 0; k < NC / 2; ++k) m.e[k] = {TC(r[2 * k]), TC(r[2 * k + 1])};
-    if (NC == 12) reconstruct_row2(m);
-    return m;
+      for (int k = 0; k < NC / 2; ++k) m.e[k] = {TC(r[2 * k]), TC(r[2 * k + 1])};
+      if (NC == 12) reconstruct_row2(m);
+      return m;
+    }
+  };
+  template <bool NT = false>
+  MAG_D Raw raw(int mu, int s) const {
+    Raw l;
+    PK::template get<NC, NT>(p, V, mu, s, l.r);
+    return l;
   }
+  template <class TC, bool NT>
+  MAG_D M3<TC> get(int mu, int s) const { return raw<NT>(mu, s).template mat<TC>(); }
   template <class TC, bool NT>
   MAG_D void put(int mu, int s, const M3<TC>& m) const {
     TS r[NC];

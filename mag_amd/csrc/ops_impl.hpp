@@ -360,16 +360,21 @@ int Ops<TS, NC>::wilson_loop(mag_ctx c, const Geom& g, void* U, const int r3[3],
     for (int i = 0; i < 3; ++i) a.r[a.nperm][i] = rl[i];
     a.nperm++;
   } while (std::next_permutation(rl, rl + 3));
-  const int nb = (g.V + BLOCK - 1) / BLOCK;
+  const int nb = (g.V + WLOOP_SITES - 1) / WLOOP_SITES;
+  // a row of the grid per permutation where the sites alone leave SIMDs idle
+  // (R = T = 4: 8^4 15 -> 9 us, 12^4 17 -> 13; 16^4 27 -> 29, 24^3 x 32 186 -> 223)
+  a.per = g.V <= SPLIT_MAX_SITES ? 1 : a.nperm;
+  const int rows = (a.nperm + a.per - 1) / a.per;
   int r;
-  if ((r = ensure_part(c, (size_t)nb))) return r;
+  if ((r = ensure_part(c, (size_t)nb * rows))) return r;
   {
     KTimer t(c, "wilson_loop");
-    hipLaunchKernelGGL((k_wilson_loop<TS, NC>), dim3(nb), dim3(BLOCK), 0, c->stream, lview<TS, NC>(U, g), a, c->d_part);
+    hipLaunchKernelGGL((k_wilson_loop<TS, NC>), dim3(nb, rows), dim3(BLOCK), 0, c->stream, lview<TS, NC>(U, g), a,
+                       c->d_part);
   }
   CHECK_LAUNCH(c);
   *nperm = a.nperm;
-  return final_reduce(c, c->d_part, nb, 1, 0, slot);
+  return final_reduce(c, c->d_part, nb * rows, 1, 0, slot);
 }
 
 }  // namespace mag
