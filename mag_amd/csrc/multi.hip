@@ -220,12 +220,18 @@ MAG_D void coarse_Q(const MultiArgs& a, const int* x0, D q[8], M3<D>& U2) {
 // and walks them with the row fastest, so the rows of one site block run
 // back to back on one XCD and the fine links they share come into its L2
 // once; the slab's neighbours along x3 are on at most two other XCDs.
-// Otherwise row-major order.
+// From 32 blocks on, nb is rounded up to a multiple of 8 for this (the surplus
+// tiles hold no sites: fine 24^4, 81 blocks, fine force 356 -> 193 us, coarse
+// force 123 -> 113); fewer blocks that do not split into 8 go row-major.
+MAG_HD int coarse_blocks(const Geom& gc) {
+  const int nb = (gc.V + BLOCK - 1) / BLOCK;
+  return nb >= 32 ? (nb + 7) / 8 * 8 : nb;
+}
 struct CTile {
   int row, blk;
 };
 MAG_D CTile ctile(const MultiArgs& a) {
-  const int nb = (a.gc.V + BLOCK - 1) / BLOCK, ny = gridDim.x / nb, b = blockIdx.x;
+  const int nb = coarse_blocks(a.gc), ny = gridDim.x / nb, b = blockIdx.x;
   if (nb % 8 == 0) {
     const int j = b >> 3;
     return {j % ny, (b & 7) * (nb >> 3) + j / ny};
@@ -503,31 +509,27 @@ struct DWalk {
   }
 };
 
+// The two rectangle staples of the plane (MU, nu) from x0 to x0 + 2 MU and
+// their derivatives, added to S and dS.
 template <int MU>
-MAG_D void cforce_link(const MultiArgs& a, const int* x0, int sc) {
-  // -i TA of Omega = stp U2^+ and of its derivative over the 6 rectangle
-  // loops (get_DQ). Every loop is a 2x1 staple from x0 to x0 + 2 mu closed by
-  // the same two links back, and the (product, derivative) step is linear in
-  // the pair, so the staples and their derivatives are summed first and the
-  // closing links applied once. The nu loop stays rolled (one nu's paths
-  // live at a time).
-  M3<D> S = zero3<D>(), dS = zero3<D>();
-#pragma unroll 1
-  for (int j = 0; j < 3; ++j) {
-    const int nu = j < MU ? j : j + 1;
-    {
-      DWalk w(a, x0);
-      w.fwd(nu); w.fwd(MU); w.fwd(MU); w.bwd(nu);
-      add_to(S, w.m);
-      add_to(dS, w.d);
-    }
-    {
-      DWalk w(a, x0);
-      w.bwd(nu); w.fwd(MU); w.fwd(MU); w.fwd(nu);
-      add_to(S, w.m);
-      add_to(dS, w.d);
-    }
+MAG_D void cforce_staples(const MultiArgs& a, const int* x0, int nu, M3<D>& S, M3<D>& dS) {
+  {
+    DWalk w(a, x0);
+    w.fwd(nu); w.fwd(MU); w.fwd(MU); w.bwd(nu);
+    add_to(S, w.m);
+    add_to(dS, w.d);
   }
+  {
+    DWalk w(a, x0);
+    w.bwd(nu); w.fwd(MU); w.fwd(MU); w.fwd(nu);
+    add_to(S, w.m);
+    add_to(dS, w.d);
+  }
+}
+
+// The coarse force of one link from the summed staples S and derivatives dS.
+template <int MU>
+MAG_D void cforce_finish(const MultiArgs& a, const int* x0, int sc, const M3<D>& S, const M3<D>& dS) {
   D q[8], dq[8];
   {
     DWalk w(a, x0);
@@ -563,6 +565,20 @@ MAG_D void cforce_link(const MultiArgs& a, const int* x0, int sc) {
 #pragma unroll
   for (int k = 0; k < 8; ++k) h[k] *= a.kappa;
   a.F.store(MU, sc, h);
+}
+
+// -i TA of Omega = stp U2^+ and of its derivative over the 6 rectangle
+// loops (get_DQ). Every loop is a 2x1 staple from x0 to x0 + 2 mu closed by
+// the same two links back, and the (product, derivative) step is linear in
+// the pair, so the staples and their derivatives are summed first and the
+// closing links applied once. The nu loop stays rolled (one nu's paths
+// live at a time).
+template <int MU>
+MAG_D void cforce_link(const MultiArgs& a, const int* x0, int sc) {
+  M3<D> S = zero3<D>(), dS = zero3<D>();
+#pragma unroll 1
+  for (int j = 0; j < 3; ++j) cforce_staples<MU>(a, x0, j < MU ? j : j + 1, S, dS);
+  cforce_finish<MU>(a, x0, sc, S, dS);
 }
 
 
@@ -618,7 +634,8 @@ __global__ __launch_bounds__(BLOCK) MAG_MULTI_OCC void k_multi_xi(MultiArgs a) {
     });
   }
   const double t = block_sum(acc);
-  if (threadIdx.x == 0) a.part[tl.row * ((a.gc.V + BLOCK - 1) / BLOCK) + tl.blk] = t;
+  const int nb = (a.gc.V + BLOCK - 1) / BLOCK;
+  if (threadIdx.x == 0 && tl.blk < nb) a.part[tl.row * nb + tl.blk] = t;
 }
 
 // simplest_metropolis with random_su3_from_su2(0.9) (field-multi-md.h:748-769,
@@ -722,16 +739,17 @@ MultiArgs args(const Multi& m, void* U, void* C, const void* xi) {
   return a;
 }
 
-int mlaunch(const Multi& m, const char* name, void (*k)(MultiArgs), dim3 grid, const MultiArgs& a) {
+int mlaunch(const Multi& m, const char* name, void (*k)(MultiArgs), dim3 grid, const MultiArgs& a,
+            int block = BLOCK) {
   if (m.c->rec) return fail(m.c, MAG_ERR_UNSUPPORTED, "the coarse/fine HMC kernels are not recordable");
   KTimer t(m.c, name);
-  hipLaunchKernelGGL(k, grid, dim3(BLOCK), 0, m.c->stream, a);
+  hipLaunchKernelGGL(k, grid, dim3(block), 0, m.c->stream, a);
   CHECK_LAUNCH(m.c);
   return MAG_OK;
 }
 
 // 1D grid of (coarse site block, row) tiles; see ctile()
-dim3 cgrid(const Multi& m, int y) { return dim3((unsigned)(((m.gc.V + BLOCK - 1) / BLOCK) * y), 1, 1); }
+dim3 cgrid(const Multi& m, int y) { return dim3((unsigned)(coarse_blocks(m.gc) * y), 1, 1); }
 
 // md::get_Fforce into F (fine alg8)
 int fforce(const Multi& m, void* F, void* U, void* C, const void* xi, const mag_action& act) {
@@ -763,11 +781,44 @@ __global__ __launch_bounds__(BLOCK) MAG_CFORCE_OCC void k_multi_cforce(MultiArgs
   with_mu(tl.row, [&](auto mc) { cforce_link<decltype(mc)::value>(a, x0, sc); });
 }
 
-// md::get_Cforce into CF (coarse alg8)
+// The same on a small coarse lattice: 64 links of one direction per block, a
+// wavefront per plane; the first sums the three pairs and finishes.
+__global__ __launch_bounds__(PLANE_THREADS) MAG_CFORCE_OCC void k_multi_cforce_split(MultiArgs a) {
+  __shared__ D red[4 * 18 * 64];
+  const int mu = blockIdx.x & 3, plane = wave_of_block();
+  const int sc = (blockIdx.x >> 2) * PLANE_SITES + (threadIdx.x & 63);
+  int x0[4];
+  coarse_site(a, min(sc, a.gc.V - 1), x0);
+  with_mu(mu, [&](auto mc) {
+    constexpr int MU = decltype(mc)::value;
+    M3<D> S = zero3<D>(), dS = zero3<D>();
+    cforce_staples<MU>(a, x0, plane < MU ? plane : plane + 1, S, dS);
+    if (plane > 0) {
+      share_put(red, 2 * plane - 2, S);
+      share_put(red, 2 * plane - 1, dS);
+    }
+    __syncthreads();
+    if (plane > 0 || sc >= a.gc.V) return;
+    for (int q = 0; q < 2; ++q) {
+      share_add(red, 2 * q, S);
+      share_add(red, 2 * q + 1, dS);
+    }
+    cforce_finish<MU>(a, x0, sc, S, dS);
+  });
+}
+
+// md::get_Cforce into CF (coarse alg8). One thread per coarse link runs one
+// wavefront per SIMD (474 registers) and leaves most SIMDs idle up to 8^4
+// coarse sites; split by planes: fine 8^4 37 -> 21 us, 12^4 54 -> 25, 16^4
+// 44 -> 33, 20^4 58 -> 70, 32^4 273 -> 308.
+constexpr int CFORCE_SPLIT_SITES = 4096;
 int cforce(const Multi& m, void* CF, void* U, void* P) {
   MultiArgs a = args(m, U, nullptr, nullptr);
   a.P = AV{(double*)P, m.gf.V};
   a.F = AV{(double*)CF, m.gc.V};
+  if (m.gc.V <= CFORCE_SPLIT_SITES)
+    return mlaunch(m, "multi_cforce", k_multi_cforce_split, dim3(4 * ((m.gc.V + PLANE_SITES - 1) / PLANE_SITES)), a,
+                   PLANE_THREADS);
   return mlaunch(m, "multi_cforce", k_multi_cforce, cgrid(m, 4), a);
 }
 
