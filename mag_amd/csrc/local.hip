@@ -19,6 +19,9 @@
 //    other x_mu parity and its staple at the other transverse parity, so
 //    the updates of one class share no staple: each class is one launch,
 //    one thread per member, and the result does not depend on thread order.
+//    Without pairs (mag = 0) the links of one transverse parity share no
+//    staple at either x_mu parity (the staple of a link holds no mu-link of
+//    another x_mu), so both parities go in one launch, with the same result.
 // Random numbers: Philox stream (seed, link, iteration); hit h of the update
 // of link (x, mu) takes draws 3h, 3h+1, 3h+2 (a, b, c, d, select, die in
 // [-1, 1), as CPS's LRG with SetInterval(1, -1)); a pair draws from its
@@ -45,7 +48,7 @@ struct LocalArgs {
   double small;
   int nhits, mag;
   uint64_t seed, iter;
-  double* cnt;   // [thread][4]: accept, reject, acceptCons, rejectCons
+  double* cnt;   // [member][4]: accept, reject, acceptCons, rejectCons (mag = 0: [member][2])
   int a, b;      // checkerboard class
 };
 
@@ -205,30 +208,74 @@ __global__ __launch_bounds__(64) void k_local_reference(LocalArgs A) {
   for (int k = 0; k < 4; ++k) A.cnt[k] = c[k];
 }
 
-// checkerboard class (MU, x_mu parity a, transverse parity b): thread t
-// enumerates the V/4 members over a lattice halved along MU and along the
-// first transverse direction T, which carries the parity fix-up.
-// Without constrained pairs (mag = 0) the kernel is held to 2 waves per SIMD
-// (20 bytes of spill; 7 % faster than 1 wave at 260 registers); the pair
-// kernel stays at 1 wave (at 2 it spills 212 bytes and is 4 % slower).
+// Members of one checkerboard launch: V/4 (x_mu parity a, transverse parity b)
+// with pairs, V/2 (transverse parity b) without.
+constexpr int LOCAL_BLOCK = 64;
+int class_members(const Geom& g, bool pair) { return g.V / (pair ? 4 : 2); }
+dim3 class_grid(const Geom& g, bool pair) {
+  return dim3(8 * (((class_members(g, pair) + 7) / 8 + LOCAL_BLOCK - 1) / LOCAL_BLOCK));
+}
+
+// Checkerboard class along MU. A member is enumerated over a lattice halved
+// along the first transverse direction T, which carries the parity fix-up, and
+// with pairs along MU too.
+//
+// What bounds it: the links of the staples. Ten hits cost less than a quarter
+// of the time at 24^4 and hide behind the loads at 32^4; with every lane two sites from
+// the next, each 128-byte line is half used by a load, and the other half
+// belongs to the member one row over. So (a) without pairs both x_mu parities
+// share a launch: the nu-links of a member at its far end are those of the
+// next member along MU at its near end, read once instead of twice; (b) an XCD
+// owns a slab of x3 and walks it with x3 faster than x2, so that rows which
+// share lines meet in one L2 (lattices whose x3 does not split in eight: a
+// contiguous eighth of the members); (c) blocks of one wavefront spread a
+// launch evenly where it is smaller than the chip. Ten hits per link, class
+// launches of an iteration, 16 of V/4 members with blocks of 256 dealt round
+// the XCDs -> now: mag = 0 8^4 327 -> 152 us, 16^4 374 -> 185, 24^4 987 -> 617,
+// 32^4 2472 -> 1687; mag = 2 (b and c only) 8^4 439 -> 445 (blocks of 256: 440), 16^4 447 -> 420,
+// 24^4 1144 -> 1002, 32^4 2906 -> 2532. Blocks of 256 in the same order: 8^4
+// 165, 16^4 196, 24^4 616, 32^4 1672 (mag = 0), 24^4 1086, 32^4 2632 (mag = 2).
+// Without pairs the kernel is held to 2 waves per SIMD (7 % faster than 1 wave
+// at 260 registers); the pair kernel stays at 1 wave (at 2 it spills 212 bytes
+// and is 4 % slower).
 template <int MU, bool PAIR>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(PAIR ? 1 : 2))) void k_local_class(LocalArgs A) {
+__global__ __launch_bounds__(LOCAL_BLOCK) __attribute__((amdgpu_waves_per_eu(PAIR ? 1 : 2))) void k_local_class(
+    LocalArgs A) {
   constexpr int T = (MU == 0) ? 1 : 0;
-  const int t = blockIdx.x * BLOCK + threadIdx.x;
-  if (t >= A.g.V / 4) return;
-  int h[4];
-  int r = t;
+  constexpr int NK = PAIR ? 4 : 2;
+  const int n = A.g.V / NK;
+  int Lh[4], h[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int Li = (i == MU || i == T) ? A.g.L[i] / 2 : A.g.L[i];
-    h[i] = r % Li;
-    r /= Li;
+  for (int i = 0; i < 4; ++i) Lh[i] = (i == T || (PAIR && i == MU)) ? A.g.L[i] / 2 : A.g.L[i];
+  const int xcd = blockIdx.x % 8;
+  const int l = (blockIdx.x / 8) * LOCAL_BLOCK + threadIdx.x;
+  int t;  // the member's count slot
+  if (Lh[3] % 8 == 0) {
+    const int w = Lh[3] / 8;
+    if (l >= n / 8) return;
+    t = xcd * (n / 8) + l;
+    int r = l;
+    h[0] = r % Lh[0];
+    r /= Lh[0];
+    h[1] = r % Lh[1];
+    r /= Lh[1];
+    h[3] = xcd * w + r % w;
+    h[2] = r / w;
+  } else {
+    t = xcd * (int)(gridDim.x / 8) * LOCAL_BLOCK + l;
+    if (t >= n) return;
+    int r = t;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      h[i] = r % Lh[i];
+      r /= Lh[i];
+    }
   }
   int x[4];
   int tr = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    if (i == MU) x[i] = 2 * h[i] + A.a;
+    if (i == MU) x[i] = PAIR ? 2 * h[i] + A.a : h[i];
     else if (i == T) x[i] = 2 * h[i];
     else {
       x[i] = h[i];
@@ -238,10 +285,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(PAIR ? 1 
   x[T] += (A.b - tr) & 1;
   double c[4];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) c[k] = A.cnt[(size_t)t * 4 + k];
+  for (int k = 0; k < NK; ++k) c[k] = A.cnt[(size_t)t * NK + k];
   update_link<PAIR>(A, x, MU, c);
 #pragma unroll
-  for (int k = 0; k < 4; ++k) A.cnt[(size_t)t * 4 + k] = c[k];
+  for (int k = 0; k < NK; ++k) A.cnt[(size_t)t * NK + k] = c[k];
 }
 
 int launch_local(mag_ctx c, void (*k)(LocalArgs), dim3 grid, dim3 block, const LocalArgs& a) {
@@ -282,14 +329,16 @@ int mag_local_metropolis(mag_field U, double beta, int mag, int num_iter, int nh
   // the reference order is one lane walking every link: a check on small lattices
   if (order == MAG_ORDER_REFERENCE && g.V > 65536)
     return fail(c, MAG_ERR_UNSUPPORTED, "the reference order runs on one lane; use it up to 16^4 sites");
-  const int nthr = order == MAG_ORDER_CHECKERBOARD ? g.V / 4 : 1;
+  const bool pair = mag > 0;
+  const int nk = order == MAG_ORDER_CHECKERBOARD && !pair ? 2 : 4;  // counts per thread
+  const int nthr = order == MAG_ORDER_CHECKERBOARD ? class_members(g, pair) : 1;
   int r;
   // per-thread hit counts, in a buffer of the shape's workspace (the
   // reductions below use the context's partial-sum buffer)
   Workspace* ws = workspace(c, g, MAG_F64, 18);
   if ((r = ws->need_cnt())) return r;
   double* cnt = (double*)ws->Cnt;
-  if ((r = fill_dev(c, cnt, 0., 4 * nthr))) return r;
+  if ((r = fill_dev(c, cnt, 0., nk * nthr))) return r;
   double* rec0 = nullptr;  // per iteration: plaquette, constrained plaquette
   if (plaq || cons_plaq) {
     if ((r = ws->need_rec(2 * (size_t)std::max(num_iter, 1)))) return r;
@@ -309,18 +358,18 @@ int mag_local_metropolis(mag_field U, double beta, int mag, int num_iter, int nh
     if (order == MAG_ORDER_REFERENCE) {
       if ((r = launch_local(c, k_local_reference, dim3(1), dim3(64), A))) return r;
     } else {
-      const dim3 grid((g.V / 4 + BLOCK - 1) / BLOCK);
+      const dim3 grid = class_grid(g, pair);
       // mag = 0 has no constrained pairs: that kernel holds one link and one
       // staple instead of two of each
       void (*kf[4])(LocalArgs) = {k_local_class<0, false>, k_local_class<1, false>, k_local_class<2, false>,
                                   k_local_class<3, false>};
       void (*kp[4])(LocalArgs) = {k_local_class<0, true>, k_local_class<1, true>, k_local_class<2, true>,
                                   k_local_class<3, true>};
-      void (**ks)(LocalArgs) = mag > 0 ? kp : kf;
+      void (**ks)(LocalArgs) = pair ? kp : kf;
       for (int mu = 0; mu < 4; ++mu)
-        for (A.a = 0; A.a < 2; ++A.a)
+        for (A.a = 0; A.a < (pair ? 2 : 1); ++A.a)
           for (A.b = 0; A.b < 2; ++A.b)
-            if ((r = launch_local(c, ks[mu], grid, dim3(BLOCK), A))) return r;
+            if ((r = launch_local(c, ks[mu], grid, dim3(LOCAL_BLOCK), A))) return r;
     }
     // reunitarize, then record the plaquette and the constrained plaquette in
     // device memory (read once after the last iteration, not per iteration)
@@ -349,10 +398,10 @@ int mag_local_metropolis(mag_field U, double beta, int mag, int num_iter, int nh
   if (acc_rej) {
     // the per-thread counts summed on the device (whole numbers: exact in
     // any order), four scalars read back
-    for (int k = 0; k < 4; ++k)
-      if ((r = final_reduce(c, cnt + k, nthr, 4, 0, k))) return r;
-    if ((r = fetch_scalars(c, 4))) return r;
-    for (int k = 0; k < 4; ++k) acc_rej[k] = (long)c->h_scalar[k];
+    for (int k = 0; k < nk; ++k)
+      if ((r = final_reduce(c, cnt + k, nthr, nk, 0, k))) return r;
+    if ((r = fetch_scalars(c, nk))) return r;
+    for (int k = 0; k < 4; ++k) acc_rej[k] = k < nk ? (long)c->h_scalar[k] : 0;
   }
   return MAG_OK;
 }
