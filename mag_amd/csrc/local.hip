@@ -25,7 +25,8 @@
 // Random numbers: Philox stream (seed, link, iteration); hit h of the update
 // of link (x, mu) takes draws 3h, 3h+1, 3h+2 (a, b, c, d, select, die in
 // [-1, 1), as CPS's LRG with SetInterval(1, -1)); a pair draws from its
-// first link. Hit counts go to per-thread slots (no atomics), summed at the end.
+// first link. Hit counts go to a slot per wavefront (no atomics), summed at the
+// end: whole numbers, so exact in any order.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -48,7 +49,7 @@ struct LocalArgs {
   double small;
   int nhits, mag;
   uint64_t seed, iter;
-  double* cnt;   // [member][4]: accept, reject, acceptCons, rejectCons (mag = 0: [member][2])
+  double* cnt;   // [block][4]: accept, reject, acceptCons, rejectCons (mag = 0: [block][2])
   int a, b;      // checkerboard class
 };
 
@@ -130,9 +131,17 @@ MAG_D M3<D> subsu2(double small, const double* u) {
 
 MAG_D double die_of(const Draws& r) { return r.u[5] < 0. ? -r.u[5] : r.u[5]; }
 
+// A hit's outcome in acc or rej: the lane's own, or (WAVE) that of all lanes
+// here, alike in each of them, so that nothing is left to sum across lanes.
+template <bool WAVE>
+MAG_D void tally(bool ok, double& acc, double& rej) {
+  acc += WAVE ? (double)__popcll(__ballot(ok)) : (ok ? 1. : 0.);
+  rej += WAVE ? (double)__popcll(__ballot(!ok)) : (ok ? 0. : 1.);
+}
+
 // One link's update (alg_gchb.h:327-368): metropolisKernel, or
 // metropolisKernelPProd with its successor for a constrained link below the last.
-template <bool PAIR>
+template <bool PAIR, bool WAVE>
 MAG_D void update_link(const LocalArgs& A, const int* x, int mu, double* c) {
   const int s = lin(A.g, x);
   const uint32_t link = (uint32_t)s * 4u + (uint32_t)mu;
@@ -160,14 +169,13 @@ MAG_D void update_link(const LocalArgs& A, const int* x, int mu, double* c) {
       const M3<D> t1 = mul(U1, eps), t2 = mul_dn(eps, U2);
       double newS = -A.fbeta * retrace_mul(t1, s1);
       newS += -A.fbeta * retrace_mul(t2, s2);
-      if (die_of(r) < exp(oldS - newS)) {
+      const bool ok = die_of(r) < exp(oldS - newS);
+      if (ok) {
         U1 = t1;
         U2 = t2;
         oldS = newS;
-        c[2] += 1.;
-      } else {
-        c[3] += 1.;
       }
+      tally<WAVE>(ok, c[2], c[3]);
     }
     A.U.store_nt(mu, s, U1);
     A.U.store_nt(mu, sy, U2);
@@ -181,13 +189,12 @@ MAG_D void update_link(const LocalArgs& A, const int* x, int mu, double* c) {
       const M3<D> eps = subsu2(A.small, r.u);
       const M3<D> t1 = mul(U, eps);
       const double newS = -A.fbeta * retrace_mul(t1, sg);
-      if (die_of(r) < exp(oldS - newS)) {
+      const bool ok = die_of(r) < exp(oldS - newS);
+      if (ok) {
         U = t1;
         oldS = newS;
-        c[0] += 1.;
-      } else {
-        c[1] += 1.;
       }
+      tally<WAVE>(ok, c[0], c[1]);
     }
     A.U.store_nt(mu, s, U);
   }
@@ -202,7 +209,7 @@ __global__ __launch_bounds__(64) void k_local_reference(LocalArgs A) {
 #pragma unroll 1
     for (int s = 0; s < A.g.V; ++s) {
       const Site p = site_of(A.g, s);
-      update_link<true>(A, p.x, mu, c);
+      update_link<true, false>(A, p.x, mu, c);
     }
 #pragma unroll
   for (int k = 0; k < 4; ++k) A.cnt[k] = c[k];
@@ -229,12 +236,15 @@ dim3 class_grid(const Geom& g, bool pair) {
 // owns a slab of x3 and walks it with x3 faster than x2, so that rows which
 // share lines meet in one L2 (lattices whose x3 does not split in eight: a
 // contiguous eighth of the members); (c) blocks of one wavefront spread a
-// launch evenly where it is smaller than the chip. Ten hits per link, class
+// launch evenly where it is smaller than the chip; (d) hits are counted by the
+// wavefront as they fall, one slot per block instead of per member (32^4 1692
+// -> 1607 us, and 0.1 ms per sum of the slots). Ten hits per link, class
 // launches of an iteration, 16 of V/4 members with blocks of 256 dealt round
-// the XCDs -> now: mag = 0 8^4 327 -> 152 us, 16^4 374 -> 185, 24^4 987 -> 617,
-// 32^4 2472 -> 1687; mag = 2 (b and c only) 8^4 439 -> 445 (blocks of 256: 440), 16^4 447 -> 420,
-// 24^4 1144 -> 1002, 32^4 2906 -> 2532. Blocks of 256 in the same order: 8^4
-// 165, 16^4 196, 24^4 616, 32^4 1672 (mag = 0), 24^4 1086, 32^4 2632 (mag = 2).
+// the XCDs -> now: mag = 0 8^4 327 -> 153 us, 16^4 374 -> 183, 24^4 987 -> 606,
+// 32^4 2472 -> 1607; mag = 2 (b to d only) 8^4 439 -> 443, 16^4 447 -> 413,
+// 24^4 1144 -> 999, 32^4 2906 -> 2454. Blocks of 256 in the same order (before
+// d): 8^4 165, 16^4 196, 24^4 616, 32^4 1672 (mag = 0), 24^4 1086, 32^4 2632
+// (mag = 2).
 // Without pairs the kernel is held to 2 waves per SIMD (7 % faster than 1 wave
 // at 260 registers); the pair kernel stays at 1 wave (at 2 it spills 212 bytes
 // and is 4 % slower).
@@ -249,11 +259,10 @@ __global__ __launch_bounds__(LOCAL_BLOCK) __attribute__((amdgpu_waves_per_eu(PAI
   for (int i = 0; i < 4; ++i) Lh[i] = (i == T || (PAIR && i == MU)) ? A.g.L[i] / 2 : A.g.L[i];
   const int xcd = blockIdx.x % 8;
   const int l = (blockIdx.x / 8) * LOCAL_BLOCK + threadIdx.x;
-  int t;  // the member's count slot
+  bool on;
   if (Lh[3] % 8 == 0) {
     const int w = Lh[3] / 8;
-    if (l >= n / 8) return;
-    t = xcd * (n / 8) + l;
+    on = l < n / 8;
     int r = l;
     h[0] = r % Lh[0];
     r /= Lh[0];
@@ -262,9 +271,8 @@ __global__ __launch_bounds__(LOCAL_BLOCK) __attribute__((amdgpu_waves_per_eu(PAI
     h[3] = xcd * w + r % w;
     h[2] = r / w;
   } else {
-    t = xcd * (int)(gridDim.x / 8) * LOCAL_BLOCK + l;
-    if (t >= n) return;
-    int r = t;
+    int r = xcd * (int)(gridDim.x / 8) * LOCAL_BLOCK + l;
+    on = r < n;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       h[i] = r % Lh[i];
@@ -283,12 +291,21 @@ __global__ __launch_bounds__(LOCAL_BLOCK) __attribute__((amdgpu_waves_per_eu(PAI
     }
   }
   x[T] += (A.b - tr) & 1;
-  double c[4];
+  // lane k keeps the block's count k
+  const int lane = threadIdx.x;
+  double* cnt = A.cnt + (size_t)blockIdx.x * NK + min(lane, NK - 1);
+  const double before = *cnt;
+  double c[4] = {0., 0., 0., 0.};
+  if (on) update_link<PAIR, true>(A, x, MU, c);
+  double mine = 0.;
 #pragma unroll
-  for (int k = 0; k < NK; ++k) c[k] = A.cnt[(size_t)t * NK + k];
-  update_link<PAIR>(A, x, MU, c);
-#pragma unroll
-  for (int k = 0; k < NK; ++k) A.cnt[(size_t)t * NK + k] = c[k];
+  for (int k = 0; k < NK; ++k) {
+    // lanes that took the other branch hold 0
+    const uint64_t took = __ballot(c[k] > 0.);
+    const double sum = __shfl(c[k], took ? __builtin_ctzll(took) : 0);
+    if (lane == k) mine = sum;
+  }
+  if (lane < NK) *cnt = before + mine;
 }
 
 int launch_local(mag_ctx c, void (*k)(LocalArgs), dim3 grid, dim3 block, const LocalArgs& a) {
@@ -330,15 +347,15 @@ int mag_local_metropolis(mag_field U, double beta, int mag, int num_iter, int nh
   if (order == MAG_ORDER_REFERENCE && g.V > 65536)
     return fail(c, MAG_ERR_UNSUPPORTED, "the reference order runs on one lane; use it up to 16^4 sites");
   const bool pair = mag > 0;
-  const int nk = order == MAG_ORDER_CHECKERBOARD && !pair ? 2 : 4;  // counts per thread
-  const int nthr = order == MAG_ORDER_CHECKERBOARD ? class_members(g, pair) : 1;
+  const int nk = order == MAG_ORDER_CHECKERBOARD && !pair ? 2 : 4;  // counts per slot
+  const int nslot = order == MAG_ORDER_CHECKERBOARD ? (int)class_grid(g, pair).x : 1;
   int r;
-  // per-thread hit counts, in a buffer of the shape's workspace (the
+  // hit counts, in a buffer of the shape's workspace (the
   // reductions below use the context's partial-sum buffer)
   Workspace* ws = workspace(c, g, MAG_F64, 18);
   if ((r = ws->need_cnt())) return r;
   double* cnt = (double*)ws->Cnt;
-  if ((r = fill_dev(c, cnt, 0., nk * nthr))) return r;
+  if ((r = fill_dev(c, cnt, 0., nk * nslot))) return r;
   double* rec0 = nullptr;  // per iteration: plaquette, constrained plaquette
   if (plaq || cons_plaq) {
     if ((r = ws->need_rec(2 * (size_t)std::max(num_iter, 1)))) return r;
@@ -396,10 +413,10 @@ int mag_local_metropolis(mag_field U, double beta, int mag, int num_iter, int nh
     }
   }
   if (acc_rej) {
-    // the per-thread counts summed on the device (whole numbers: exact in
+    // the counts summed on the device (whole numbers: exact in
     // any order), four scalars read back
     for (int k = 0; k < nk; ++k)
-      if ((r = final_reduce(c, cnt + k, nthr, nk, 0, k))) return r;
+      if ((r = final_reduce(c, cnt + k, nslot, nk, 0, k))) return r;
     if ((r = fetch_scalars(c, nk))) return r;
     for (int k = 0; k < 4; ++k) acc_rej[k] = k < nk ? (long)c->h_scalar[k] : 0;
   }

@@ -267,7 +267,7 @@ struct Workspace {
   void* Utop = nullptr;  // FP64 12-real chains: the force's top smeared level, 18 reals
   void* Lam = nullptr;  // alg8: Lambda of the coarse/fine HMC (coarse shape)
   void* Eq = nullptr;   // mat18: e^{iQ} of the coarse/fine HMC (coarse shape)
-  void* Cnt = nullptr;  // V doubles: per-thread hit counts of the local Metropolis
+  void* Cnt = nullptr;  // max(V, 32) doubles: hit counts of the local updates
   void* Rec = nullptr;  // per-iteration records of the local Metropolis (grows)
   size_t rec_cap = 0;
 
@@ -307,7 +307,7 @@ struct Workspace {
   }
   int need_Z() { return get(&Z, mat_bytes()); }
   int need_top18() { return get(&Utop, mat64_bytes()); }
-  int need_cnt() { return get(&Cnt, (size_t)g.V * sizeof(double)); }
+  int need_cnt() { return get(&Cnt, std::max((size_t)g.V, (size_t)32) * sizeof(double)); }
   int need_rec(size_t n) {
     if (Rec && rec_cap >= n) return MAG_OK;
     if (Rec) {
