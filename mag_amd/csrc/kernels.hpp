@@ -781,6 +781,7 @@ MAG_D void k_stout_top_tile_body(const StoutTopArgs<float, 12, 12>& a) {
   stencil_tile<false>(a.g, mu, sblk);
   const int L0 = a.g.L[0], L1 = a.g.L[1], plane = L0 * L1;
   const int s0 = sblk * BLOCK;
+  if (s0 >= a.g.V) return;  // a surplus block of the rounded-up grid (the shape has whole blocks only)
   const int sl = s0 - s0 % plane;  // first site of the (x2, x3) slice
   const int x1lo = (s0 - sl) / L0;
   const int nt = BLOCK + 4 * L0;
