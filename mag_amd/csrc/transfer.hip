@@ -120,41 +120,28 @@ __global__ __launch_bounds__(TB) void k_real_from_host(double* p, int V, int s0,
 }
 
 template <class TS, int NC, bool ALG>
-void launch_matrix(mag_field f, bool down, int s0, int ns, double* slot) {
-  const dim3 grid((ns + 63) / 64);
-  if (down)
-    hipLaunchKernelGGL((k_to_host<TS, NC, ALG>), grid, dim3(TB), 0, f->ctx->stream, (TS*)f->p, f->g.V, s0, ns, slot);
-  else
-    hipLaunchKernelGGL((k_from_host<TS, NC, ALG>), grid, dim3(TB), 0, f->ctx->stream, (TS*)f->p, f->g.V, s0, ns,
-                       (const double*)slot);
+const void* matrix_kernel(bool down) {
+  return down ? (const void*)k_to_host<TS, NC, ALG> : (const void*)k_from_host<TS, NC, ALG>;
 }
 
-// Sites [s0, s0 + ns) of f to (from) a pinned slot.
+// Sites [s0, s0 + ns) of f to (from) a pinned slot. Answers with the launch's
+// own status: the thread's last error may have been left by an earlier call.
 hipError_t launch_chunk(mag_field f, bool down, int s0, int ns, double* slot) {
   const bool f64 = f->prec == MAG_F64;
+  const void* k = nullptr;
+  int nb = (ns + 63) / 64;
   switch (f->kind) {
-    case MAG_REAL1: {
-      const dim3 grid((4 * ns + TB - 1) / TB);
-      if (down)
-        hipLaunchKernelGGL(k_real_to_host, grid, dim3(TB), 0, f->ctx->stream, (const double*)f->p, f->g.V, s0, ns,
-                           slot);
-      else
-        hipLaunchKernelGGL(k_real_from_host, grid, dim3(TB), 0, f->ctx->stream, (double*)f->p, f->g.V, s0, ns,
-                           (const double*)slot);
+    case MAG_REAL1:
+      k = down ? (const void*)k_real_to_host : (const void*)k_real_from_host;
+      nb = (4 * ns + TB - 1) / TB;
       break;
-    }
-    case MAG_ALG8:
-      if (f64) launch_matrix<double, 8, true>(f, down, s0, ns, slot);
-      else launch_matrix<float, 8, true>(f, down, s0, ns, slot);
-      break;
-    case MAG_LINK12:
-      if (f64) launch_matrix<double, 12, false>(f, down, s0, ns, slot);
-      else launch_matrix<float, 12, false>(f, down, s0, ns, slot);
-      break;
-    default:
-      launch_matrix<double, 18, false>(f, down, s0, ns, slot);  // MAG_LINK18 fields are FP64
+    case MAG_ALG8: k = f64 ? matrix_kernel<double, 8, true>(down) : matrix_kernel<float, 8, true>(down); break;
+    case MAG_LINK12: k = f64 ? matrix_kernel<double, 12, false>(down) : matrix_kernel<float, 12, false>(down); break;
+    default: k = matrix_kernel<double, 18, false>(down);  // MAG_LINK18 fields are FP64
   }
-  return hipGetLastError();
+  int V = f->g.V;
+  void* args[] = {&f->p, &V, &s0, &ns, &slot};
+  return hipLaunchKernel(k, dim3(nb), dim3(TB), args, 0, f->ctx->stream);
 }
 
 // The context's pinned slots and their events, grown to what a call needs.
