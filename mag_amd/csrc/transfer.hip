@@ -144,6 +144,24 @@ hipError_t launch_chunk(mag_field f, bool down, int s0, int ns, double* slot) {
   return hipLaunchKernel(k, dim3(nb), dim3(TB), args, 0, f->ctx->stream);
 }
 
+// The calling thread on the context's device for the length of a call: pinned
+// slots and events are made on the current device, and an event of another
+// device is refused on the context's stream. The caller's device is put back.
+struct OnDevice {
+  int before = -1;
+  hipError_t status;
+  explicit OnDevice(int device) {
+    int d = device;
+    status = hipGetDevice(&d);
+    if (status != hipSuccess || d == device) return;
+    status = hipSetDevice(device);
+    if (status == hipSuccess) before = d;
+  }
+  ~OnDevice() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+};
+
 // The context's pinned slots and their events, grown to what a call needs.
 int need_stage(mag_ctx c, size_t bytes, size_t events) {
   if (bytes > c->stage_cap) {
@@ -173,6 +191,8 @@ namespace mag {
 int field_transfer(mag_field f, double* host, bool down) {
   mag_ctx c = f->ctx;
   const std::lock_guard<std::mutex> hold(c->stage_mu);
+  const OnDevice here(c->device);
+  HIPCHK(c, here.status);
   const size_t per = (f->kind == MAG_REAL1 ? 4 : ROW) * sizeof(double), total = per * (size_t)f->g.V;
   // about eight chunks, 512 KiB (35 GB/s over the link; less is latency) to 4 MiB (50 GB/s) each
   const size_t want = std::min(std::max(total / 8, CHUNK_MIN), CHUNK_MAX);
@@ -186,7 +206,10 @@ int field_transfer(mag_field f, double* host, bool down) {
   std::atomic<int> bad{(int)hipSuccess};
   std::atomic<int> next{0};
   auto work = [&](int w) {
-    if (w) (void)hipSetDevice(c->device);  // a new thread starts on device 0
+    if (w) {  // a new thread starts on device 0
+      const hipError_t e = hipSetDevice(c->device);
+      if (e != hipSuccess) bad = (int)e;
+    }
     char* slot[2] = {c->stage + slot_bytes * (2 * w), c->stage + slot_bytes * (2 * w + 1)};
     const hipEvent_t ev[2] = {c->stage_ev[2 * w], c->stage_ev[2 * w + 1]};
     int held[2] = {-1, -1};  // chunk in flight in each slot

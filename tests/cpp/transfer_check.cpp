@@ -156,6 +156,20 @@ static int round_trip(Rig& rig, const int L[4], int kind, int current) {
 
 static const int SHAPES[][4] = {{4, 4, 4, 4}, {5, 7, 4, 9}, {8, 8, 8, 8}, {9, 7, 11, 13}, {16, 16, 16, 20}, {32, 32, 32, 8}};
 
+// A context of device 1, called from threads whose current device is 0 or 1.
+static int check_device() {
+  for (const auto& L : SHAPES)
+    for (int kind : {(int)MAG_REAL1, (int)MAG_LINK18})
+      for (int current : {0, 1}) {
+        Rig rig;
+        if (round_trip(rig, L, kind, current)) return 1;
+        REQUIRE(!g_bad_alloc && !g_bad_event && !g_bad_launch, "%d allocations, %d events, %d launches off the device",
+                g_bad_alloc, g_bad_event, g_bad_launch);
+      }
+  std::printf("ok device\n");
+  return 0;
+}
+
 // A transfer answers for its own launches: an error that an earlier call left
 // behind is none of its, a launch that fails is.
 static int check_error() {
@@ -178,6 +192,7 @@ static int check_error() {
 
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "device") return check_device();
   if (what == "error") return check_error();
   return 2;
 }
