@@ -196,7 +196,7 @@ int field_transfer(mag_field f, double* host, bool down) {
   const size_t per = (f->kind == MAG_REAL1 ? 4 : ROW) * sizeof(double), total = per * (size_t)f->g.V;
   // about eight chunks, 512 KiB (35 GB/s over the link; less is latency) to 4 MiB (50 GB/s) each
   const size_t want = std::min(std::max(total / 8, CHUNK_MIN), CHUNK_MAX);
-  const int step = (int)((want / per + 63) / 64 * 64);
+  const int step = (int)(std::min((want / per + 63) / 64, CHUNK_MAX / per / 64) * 64);  // whole blocks of 64 sites
   const int nchunk = (f->g.V + step - 1) / step;
   // one more thread (11 us to start) per 2 MiB: two slots each
   const int workers = (int)std::min<size_t>({(size_t)WORKERS_MAX, (total + (2 << 20) - 1) / (2 << 20), (size_t)nchunk});

@@ -190,9 +190,28 @@ static int check_error() {
   return 0;
 }
 
+// The pinned memory that a context holds after fields of any size.
+static int check_bound() {
+  const int shapes[][4] = {{4, 4, 4, 4}, {9, 7, 11, 13}, {16, 16, 16, 20}, {24, 24, 24, 32}, {32, 32, 32, 32}};
+  for (const auto& L : shapes)
+    for (int kind : {(int)MAG_REAL1, (int)MAG_LINK18}) {
+      Rig rig;
+      std::vector<double> store;
+      mag_field_s f = field(rig, L, kind, store);
+      std::unique_ptr<double[]> host(new double[(size_t)f.g.V * (kind == MAG_REAL1 ? 4 : ROW)]);
+      g_pinned_max = 0;
+      REQUIRE(field_transfer(&f, host.get(), true) == MAG_OK, "download refused");
+      if (moved_once(f)) return 1;
+      REQUIRE(g_pinned_max <= (size_t)32 << 20, "%zu bytes pinned for %d sites of kind %d", g_pinned_max, f.g.V, kind);
+    }
+  std::printf("ok bound\n");
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "device") return check_device();
   if (what == "error") return check_error();
+  if (what == "bound") return check_bound();
   return 2;
 }

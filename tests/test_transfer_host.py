@@ -1,7 +1,7 @@
 """Field transfers on the CPU, over a stand-in for the HIP runtime
 (tests/cpp/transfer_check.cpp): every site moved once, whatever device the
 calling thread is on; errors that earlier calls left behind not taken for the
-transfer's own."""
+transfer's own; at most 32 MiB of pinned slots."""
 import os
 import shutil
 import subprocess
@@ -22,7 +22,7 @@ def exe(tmp_path_factory):
     return str(out)
 
 
-@pytest.mark.parametrize("check", ["device", "error"])
+@pytest.mark.parametrize("check", ["device", "error", "bound"])
 def test_transfers(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
