@@ -7,7 +7,6 @@ are handles; host arrays use the reference's qlat layout, float64 of shape
 (V, 4, 18) = [site][mu][3x3 complex, interleaved re/im].
 """
 import ctypes as C
-import weakref
 from dataclasses import dataclass, field as dfield
 
 import numpy as np
@@ -50,7 +49,11 @@ class Context:
 
     def __init__(self, device=0):
         self._h = C.c_void_p()
-        self._children = weakref.WeakSet()  # fields, chains, servers created on this context
+        # Fields, chains and servers created on this context, in order: the handle and what destroys it. The
+        # handles themselves, not weak references to their owners: those are cleared before any __del__ when the
+        # garbage collector takes the context and its objects together.
+        self._live = {}
+        self._destroy = _lib.lib().mag_ctx_destroy
         _check(_lib.lib().mag_ctx_create(device, C.byref(self._h)))
 
     @property
@@ -58,15 +61,22 @@ class Context:
         return self._h
 
     def adopt(self, obj):
-        self._children.add(obj)
+        self._live[id(obj._h)] = (obj._h, getattr(_lib.lib(), obj._destroy))
+
+    def release(self, handle):
+        """Destroy an adopted object, once; its handle is null from then on."""
+        h, destroy = self._live.pop(id(handle), (None, None))
+        if h:
+            destroy(h)
+            h.value = None
 
     def close(self):
         """Destroy the context after every live object created on it (the C ABI
         requires fields, chains and servers to go first)."""
         if self._h:
-            for ch in list(self._children):
-                ch._release()
-            _lib.lib().mag_ctx_destroy(self._h)
+            for h, _ in reversed(list(self._live.values())):
+                self.release(h)
+            self._destroy(self._h)
             self._h = C.c_void_p()
 
     def __del__(self):
@@ -99,17 +109,32 @@ class Context:
         return ms.value, n.value
 
 
-class Field:
+class _Adopted:
+    """An object that its context (self.ctx) destroys if it is still there when the context goes."""
+
+    def _release(self):
+        self.ctx.release(self._h)
+
+    def __del__(self):
+        try:
+            self._release()
+        except Exception:
+            pass
+
+
+class Field(_Adopted):
     """Device field (qlat::Field<cps::Matrix> of multiplicity 4)."""
+
+    _destroy = "mag_field_destroy"
 
     def __init__(self, ctx, dims, kind=LINK18, prec=F64, _handle=None):
         self.ctx = ctx
         self.dims = tuple(int(d) for d in dims)
         self.kind, self.prec = kind, prec
         if _handle is not None:
-            self._h, self._owned = _handle, False
+            self._h = _handle  # borrowed: never adopted, so never destroyed here
         else:
-            self._h, self._owned = C.c_void_p(), True
+            self._h = C.c_void_p()
             _check(_lib.lib().mag_field_create(ctx.handle, (C.c_int * 4)(*self.dims), kind, prec, C.byref(self._h)),
                    ctx.handle)
             ctx.adopt(self)
@@ -121,17 +146,6 @@ class Field:
     @property
     def volume(self):
         return int(np.prod(self.dims))
-
-    def _release(self):
-        if self._owned and self._h:
-            _lib.lib().mag_field_destroy(self._h)
-        self._h = C.c_void_p()
-
-    def __del__(self):
-        try:
-            self._release()
-        except Exception:
-            pass
 
     def _host_shape(self):
         # REAL1: one real per link ([site][mu]); otherwise 3x3 complex per link
@@ -422,8 +436,10 @@ class AlgGCtrnHeatBath:
 
 
 # ----------------------------------------------------------------- chain
-class Chain:
+class Chain(_Adopted):
     """Device-resident HMC chain (run_chmc / update_field, field-hmc.h:770-986)."""
+
+    _destroy = "mag_chain_destroy"
 
     def __init__(self, ctx, dims, arg, seed=1234, precision=F64, integrator=0, accept_mode=0, demon_emax=0.0,
                  reunit=True, recon12=None):
@@ -439,17 +455,6 @@ class Chain:
         _check(_lib.lib().mag_chain_create(ctx.handle, (C.c_int * 4)(*self.dims), C.byref(self.act),
                                            C.byref(self.params), C.byref(self._h)), ctx.handle)
         ctx.adopt(self)
-
-    def _release(self):
-        if self._h:
-            _lib.lib().mag_chain_destroy(self._h)
-        self._h = C.c_void_p()
-
-    def __del__(self):
-        try:
-            self._release()
-        except Exception:
-            pass
 
     def set_links(self, host):
         a = np.ascontiguousarray(host, dtype=np.float64)

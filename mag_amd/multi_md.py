@@ -12,7 +12,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import ALG8, F64, LINK18, REAL1, HmcParams, MultiParams, MultiResult
-from . import Field, _act, _check, _dptr
+from . import Field, _act, _Adopted, _check, _dptr
 
 MD_ALPHA = 0.5
 ZETA_H, FG, NESTED = 0, 1, 2
@@ -124,8 +124,10 @@ def get_hamiltonian_multi(FgField, FmField, Farg, CgField, CxField, mp):
     return h.value, parts
 
 
-class MultiChain:
+class MultiChain(_Adopted):
     """md::run_hmc_multi (field-multi-md.h:785-988) as a device-resident chain."""
+
+    _destroy = "mag_multi_destroy"
 
     def __init__(self, ctx, dims, Farg, mp, seed=1234):
         self.ctx = ctx
@@ -138,17 +140,6 @@ class MultiChain:
         _check(_lib.lib().mag_multi_create(ctx.handle, (C.c_int * 4)(*self.dims), C.byref(self.act),
                                            C.byref(self.params), C.byref(mp), C.byref(self._h)), ctx.handle)
         ctx.adopt(self)
-
-    def _release(self):
-        if self._h:
-            _lib.lib().mag_multi_destroy(self._h)
-        self._h = C.c_void_p()
-
-    def __del__(self):
-        try:
-            self._release()
-        except Exception:
-            pass
 
     def fields(self):
         """Borrowed (fine, coarse) link fields of the chain."""

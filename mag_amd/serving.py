@@ -12,7 +12,7 @@ import time
 
 import numpy as np
 
-from . import _lib
+from . import _Adopted, _lib
 from ._lib import F32, F64, IWASAKI, WILSON, Action, HmcParams, ServeRequest, TrajResult
 
 STATE = {0: "pending", 1: "running", 2: "done", 3: "failed", 4: "cancelled"}
@@ -38,7 +38,9 @@ def footprint(req):
     return b.value
 
 
-class Server:
+class Server(_Adopted):
+    _destroy = "mag_server_destroy"
+
     def __init__(self, ctx, hbm_budget=64 << 30, max_batch=64, graphs=True):
         self.ctx = ctx
         self._h = C.c_void_p()
@@ -47,19 +49,8 @@ class Server:
         ctx.adopt(self)
         self.ntraj = {}
 
-    def _release(self):
-        if self._h:
-            _lib.lib().mag_server_destroy(self._h)
-        self._h = C.c_void_p()
-
     def close(self):
         self._release()
-
-    def __del__(self):
-        try:
-            self.close()
-        except Exception:
-            pass
 
     def submit(self, req):
         i = C.c_int()
