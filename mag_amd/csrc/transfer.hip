@@ -84,11 +84,18 @@ __global__ __launch_bounds__(TB) void k_from_host(TS* p, int V, int s0, int ns, 
   const int lane = threadIdx.x & 63, mu = threadIdx.x >> 6, b0 = blockIdx.x * 64;
   const int n2 = min(64, ns - b0) * (ROW / 2);
   const V2* src = (const V2*)(in + (size_t)b0 * ROW);
-  for (int i = threadIdx.x; i < n2; i += TB) {
-    const int site = i / (ROW / 2), c = 2 * (i - site * (ROW / 2));
-    const V2 v = src[i];
-    buf[site * LROW + c] = v[0];
-    buf[site * LROW + c + 1] = v[1];
+  // all loads over the link on their way at once (one by one 6 us more per call: 4^4 links 26.8 -> 20.7)
+  constexpr int PER = 64 * (ROW / 2) / TB;
+  V2 v[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+    if ((int)threadIdx.x + k * TB < n2) v[k] = src[threadIdx.x + k * TB];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = threadIdx.x + k * TB, site = i / (ROW / 2), c = 2 * (i - site * (ROW / 2));
+    if (i >= n2) break;
+    buf[site * LROW + c] = v[k][0];
+    buf[site * LROW + c + 1] = v[k][1];
   }
   __syncthreads();
   if (b0 + lane >= ns) return;
