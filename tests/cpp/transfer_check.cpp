@@ -1,9 +1,9 @@
 // Host-side check of field transfers (transfer.hip) over a HIP runtime that
 // this program stands in for: two devices, a current device per thread,
 // streams and events that belong to a device (recording an event on another
-// device's stream is refused, as by the runtime), and kernels that are
-// emulated for one-real-per-link fields and write (or check) the site number
-// for link fields. argv[1] names the check; prints "ok" lines and exits
+// device's stream is refused, as by the runtime), copies, and kernels that are
+// emulated for one-real-per-link fields and write the site number for link
+// fields. argv[1] names the check; prints "ok" lines and exits
 // non-zero on the first violation.
 #include "../../mag_amd/csrc/transfer.hip"
 
@@ -65,6 +65,12 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 
+hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t) {
+  if (g_launch != hipSuccess) return g_launch;
+  std::memcpy(dst, src, n);
+  for (int& s : g_sites) ++s;  // whole fields only
+  return hipSuccess;
+}
 hipError_t hipLaunchKernel(const void* k, dim3, dim3, void** args, size_t, hipStream_t s) {
   if (g_launch != hipSuccess) return g_launch;
   const int V = *(int*)args[1], s0 = *(int*)args[2], ns = *(int*)args[3];
@@ -118,6 +124,7 @@ static mag_field_s field(Rig& rig, const int L[4], int kind, std::vector<double>
   f.g = make_geom(L);
   store.resize(kind == MAG_REAL1 ? (size_t)f.g.V * 4 : 1);  // link values are not looked at
   f.p = store.data();
+  f.bytes = store.size() * sizeof(double);
   g_sites.assign((size_t)f.g.V, 0);
   return f;
 }
