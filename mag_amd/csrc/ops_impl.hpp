@@ -52,18 +52,21 @@ int Ops<TS, NC>::link_update(mag_ctx c, const Geom& g, void* Uin, void* Uout, vo
   return launch(c, "link_update", k_link_update<TS, NC, TS, R12>, k_link_update_b<TS, NC, TS, R12>, grid_links(g), a);
 }
 
-// Thin-link force. Constrained runs: up to SPLIT_MAX_SITES the links with two
+// Thin-link force. Constrained runs on small lattices: the links with two
 // staple sums have blocks of their own, since with both sums in the stencil
 // every wavefront that meets such a link is twice as long (FP64 Iwasaki, mag
 // = 2: 4^4 58 -> 22 us, 8^4 61 -> 24, 12^4 107 -> 60; FP32 61 -> 17, 65 -> 18,
 // 64 -> 27). On larger lattices that costs little, and those blocks, which
 // share no neighbours with the stencil's in flight, cost more: 32^4 2.44 ms in
-// one thread per link, 2.86 with them.
+// one thread per link, 2.86 with them. Block size 1 has no such link and no force
+// at all (the classes alone say so: 5 us against 45 at 12^4), and a negative size,
+// whose links are never the last of a block, is not one that pair_site lists.
+inline bool gather_pairs(const Geom& g, int mag) { return mag >= 2 && g.V <= SPLIT_MAX_SITES; }
 template <int ACT, class TS, int NC>
 int thin_force(mag_ctx c, ForceArgs<TS, NC> fa) {
   const char* name = ACT == ACT_IWASAKI ? "force_iwasaki" : "force_wilson";
   const Geom& g = fa.g;
-  if (fa.mag && g.V > SPLIT_MAX_SITES)
+  if (fa.mag && !gather_pairs(g, fa.mag))
     return launch(c, name, k_gauge_force<ACT, true, TS, NC, TS>, k_gauge_force_b<ACT, true, TS, NC, TS>,
                   grid_stencil(g), fa);
   if (fa.mag) {
