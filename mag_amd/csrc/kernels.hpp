@@ -95,8 +95,8 @@ MAG_D void stencil_tile(const Geom& g, int& mu, int& sblk) {
 // LDS in plane order, and the first of them goes on alone with what follows
 // the sum. Rules and measurements at launch_stencil().
 //
-// A stencil K has Args (with Geom g), Real, waves (per SIMD),
-// share(args, site, mu, plane) and finish(args, mu, s, sum).
+// A stencil K has Args (with Geom g), Real, waves (per SIMD), smears (a long
+// finish), share(args, site, mu, plane) and finish(args, mu, s, sum).
 constexpr int PLANE_SITES = 64, PLANE_THREADS = 3 * PLANE_SITES;
 
 template <class TC>
@@ -423,6 +423,7 @@ template <int ACT, bool CONS, class TS, int NC, class TC>
 struct ForceStencil {
   using Args = ForceArgs<TS, NC>;
   using Real = TC;
+  static constexpr bool smears = false;
   static constexpr int waves = stencil_waves<TC>();
   MAG_D static M3<TC> share(const Args& a, const Site& p, int mu, int plane) {
     const TC c1 = (ACT == ACT_IWASAKI) ? TC(a.c1) : TC(0);
@@ -624,6 +625,7 @@ template <class TSI, int NCI, class TSO, int NCO, class TC, bool R12 = false>
 struct FwdStencil {
   using Args = StoutFwdArgs<TSI, NCI, TSO, NCO>;
   using Real = TC;
+  static constexpr bool smears = true;
   static constexpr int waves = stencil_waves<TC>();
   MAG_D static M3<TC> share(const Args& a, const Site& p, int mu, int plane) {
     if constexpr (R12) return staple_share<ACT_WILSON, TC>(SU3Read<TSI, NCI>{a.U}, a.g, p, mu, plane, TC(1), TC(0));
@@ -690,6 +692,7 @@ template <int ACT, class TS, int NC, class TC, int NCN = NC>
 struct TopStencil {
   using Args = StoutTopArgs<TS, NC, NCN>;
   using Real = TC;
+  static constexpr bool smears = true;
   static constexpr int waves = stencil_waves<TC>();
   MAG_D static M3<TC> share(const Args& a, const Site& p, int mu, int plane) {
     const TC c1 = (ACT == ACT_IWASAKI) ? TC(a.c1) : TC(0);
@@ -985,6 +988,7 @@ template <bool LAST, class TS, int NC, class TC, bool R12 = false>
 struct BwdStencil {
   using Args = StoutBwdArgs<TS, NC>;
   using Real = TC;
+  static constexpr bool smears = true;
   static constexpr int waves = stencil_waves<TC>();
   MAG_D static M3<TC> share(const Args& a, const Site& p, int mu, int plane) {
     M3<TC> acc = zero3<TC>();
@@ -1323,6 +1327,7 @@ struct WloopArgs {
   int T;
 };
 constexpr int WLOOP_SITES = BLOCK / 2;
+constexpr int WLOOP_ROW_SITES = 1 << 15;
 // Block of WLOOP_SITES sites that block b of nb takes: XCD k (b mod 8) has a
 // contiguous run of a walk with x3 fastest where an x3 slice is whole blocks
 // (the temporal lines of the sites that share them then meet in its L2: 24^3 x

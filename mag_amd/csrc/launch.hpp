@@ -74,20 +74,37 @@ template <class A, class K>
 int launch_split(mag_ctx c, const char* timer, Stencil<K>, const Geom& g, const A& a) {
   return launch(c, timer, k_split<K>, k_split_b<K>, grid_split(g), a, PLANE_THREADS);
 }
-// The split form up to SPLIT_MAX_SITES, else one thread per link (ks, kb). An
-// Iwasaki + 3-stout force, back to back, one thread per link -> split:
-//   FP32   4^4 88 -> 49 us, 8^4 92 -> 55, 10^4 102 -> 75, 12^4 120 -> 115, 14^4 176 -> 176, 16^4 257 -> 280
-//   FP64   4^4 119 -> 65,   8^4 135 -> 79, 10^4 147 -> 133, 12^4 232 -> 213, 14^4 371 -> 328
+// The split form up to a number of sites, else one thread per link (ks, kb).
 // Below the line one thread per link leaves most SIMDs with one wavefront or
 // none; above it all are busy either way, and two of three wavefronts idle
-// while the first goes on costs 5-15 %. Six wavefronts (plane and side) took
-// 50 us at FP32 8^4 but 149 at 12^4; three groups of sites per block, every
-// wavefront going on with one, gave the split's gain back.
-constexpr int SPLIT_MAX_SITES = 1 << 15;
+// while the first goes on costs 5-30 %. Iwasaki + 3-stout force, back to back,
+// one thread per link -> split:
+//   FP32   8^4 93 -> 57 us, 10^4 100 -> 71, 12^4 117 -> 113, 27,648 sites 122 -> 136, 32,768 134 -> 151
+//   FP64   8^4 119 -> 93,   10^4 134 -> 130, 12^4 212 -> 212, 27,648 sites 238 -> 256, 32,768 276 -> 293
+// Time of the split form over that of one thread per link, by sites:
+//                               8,192  12,288  16,384  18,432  20,736  24,576  28,672  32,768
+//   FP32 Wilson + 3-stout force   0.65    0.77    0.81    0.87    0.97    1.05    1.13    1.14
+//   FP32 smearing                 0.65    0.76    0.82    0.83    1.02    1.04    1.14    1.15
+//   FP64 Wilson + 3-stout force   0.74    1.01    1.19    0.92    0.99    1.08    1.12    1.10
+//   FP64 smearing                 0.76    1.04    1.28    0.96    1.01    1.16    1.22    1.06
+//   FP64 thin Wilson force        0.70    0.85    0.96    0.77    0.83    0.93    0.97    0.80
+//   FP64 thin, 12-real links      0.74    0.88    0.95    0.84    0.93    0.98    1.02    1.06
+// FP64 one thread per link takes as long for any lattice up to 16,384 sites (one
+// wavefront per SIMD) and nearly twice that from there; the split form, two blocks
+// per CU, needs a second round from 8,192. Six wavefronts (plane and side) took 50
+// us at FP32 8^4 but 149 at 12^4; three groups of sites per block, every wavefront
+// going on with one, gave the split's gain back.
+constexpr int SPLIT_MAX_SITES = 20736;  // 12^4
+template <class K>
+constexpr bool split_wins(int V) {
+  if (sizeof(typename K::Real) == sizeof(float)) return V <= SPLIT_MAX_SITES;
+  if (!K::smears) return V <= 24576;
+  return V <= 8192 || (V > 16384 && V <= SPLIT_MAX_SITES);
+}
 template <class A, class K>
 int launch_stencil(mag_ctx c, const char* timer, void (*ks)(A), void (*kb)(const A*), Stencil<K> k, const Geom& g,
                    const A& a) {
-  if (g.V <= SPLIT_MAX_SITES) return launch_split(c, timer, k, g, a);
+  if (split_wins<K>(g.V)) return launch_split(c, timer, k, g, a);
   return launch(c, timer, ks, kb, grid_stencil(g), a);
 }
 

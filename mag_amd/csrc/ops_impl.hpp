@@ -29,7 +29,8 @@ namespace mag {
 template <class TS, int NC>
 constexpr bool ops_read12(int bit) { return (MAG_FP64_READ12 & bit) != 0 && std::is_same<TS, double>::value && NC == 18; }
 
-// FP64 rectangle staples always take the split form. One thread per link
+// FP64 rectangle staples take the split form (with one exception in
+// thin_force). One thread per link
 // needs more than 256 VGPRs for them (it spills, or runs one wave per SIMD),
 // a plane's share fits; and three wavefronts on the same 64 sites ask L2 for
 // a third of the sites at a time. Thin force / top kernel, one thread per
@@ -58,15 +59,19 @@ int Ops<TS, NC>::link_update(mag_ctx c, const Geom& g, void* Uin, void* Uout, vo
 // = 2: 4^4 58 -> 22 us, 8^4 61 -> 24, 12^4 107 -> 60; FP32 61 -> 17, 65 -> 18,
 // 64 -> 27). On larger lattices that costs little, and those blocks, which
 // share no neighbours with the stencil's in flight, cost more: 32^4 2.44 ms in
-// one thread per link, 2.86 with them. Block size 1 has no such link and no force
-// at all (the classes alone say so: 5 us against 45 at 12^4), and a negative size,
+// one thread per link, 2.86 with them; FP64 Wilson at 28,672 sites 1.08 of one
+// thread per link (at 27,648 0.98). Block size 1 has no such link and no force at
+// all (the classes alone say so: 5 us against 45 at 12^4), and a negative size,
 // whose links are never the last of a block, is not one that pair_site lists.
-inline bool gather_pairs(const Geom& g, int mag) { return mag >= 2 && g.V <= SPLIT_MAX_SITES; }
+template <int ACT, class TS>
+bool gather_pairs(const Geom& g, int mag) {
+  return mag >= 2 && g.V <= (ACT == ACT_WILSON && std::is_same<TS, double>::value ? 24576 : 32768);
+}
 template <int ACT, class TS, int NC>
 int thin_force(mag_ctx c, ForceArgs<TS, NC> fa) {
   const char* name = ACT == ACT_IWASAKI ? "force_iwasaki" : "force_wilson";
   const Geom& g = fa.g;
-  if (fa.mag && !gather_pairs(g, fa.mag))
+  if (fa.mag && !gather_pairs<ACT, TS>(g, fa.mag))
     return launch(c, name, k_gauge_force<ACT, true, TS, NC, TS>, k_gauge_force_b<ACT, true, TS, NC, TS>,
                   grid_stencil(g), fa);
   if (fa.mag) {
@@ -78,10 +83,16 @@ int thin_force(mag_ctx c, ForceArgs<TS, NC> fa) {
     return launch(c, name, k_cons_force<ACT, TS, NC, TS>, k_cons_force_b<ACT, TS, NC, TS>, grid, fa, PLANE_THREADS);
   }
   const Stencil<ForceStencil<ACT, false, TS, NC, TS>> split;
-  if constexpr (ACT == ACT_IWASAKI && split_rectangles<TS>()) return launch_split(c, name, split, g, fa);
-  else
+  if constexpr (ACT == ACT_IWASAKI && split_rectangles<TS>()) {
+    // 12-real links: one wavefront per SIMD takes 27-28 us up to
+    // 16,384 sites; split 24.6 at 12,288, 29.9 at 13,824, 30.9 at 16,384
+    if (NC != 12 || g.V <= 12288 || g.V > 16384) return launch_split(c, name, split, g, fa);
+    return launch(c, name, k_gauge_force<ACT, false, TS, NC, TS>, k_gauge_force_b<ACT, false, TS, NC, TS>,
+                  grid_stencil(g), fa);
+  } else {
     return launch_stencil(c, name, k_gauge_force<ACT, false, TS, NC, TS>, k_gauge_force_b<ACT, false, TS, NC, TS>,
                           split, g, fa);
+  }
 }
 
 // Force of the (possibly smeared) action on U with one of the epilogues
@@ -366,7 +377,7 @@ int Ops<TS, NC>::wilson_loop(mag_ctx c, const Geom& g, void* U, const int r3[3],
   const int nb = (g.V + WLOOP_SITES - 1) / WLOOP_SITES;
   // a row of the grid per permutation where the sites alone leave SIMDs idle
   // (R = T = 4: 8^4 15 -> 9 us, 12^4 17 -> 13; 16^4 27 -> 29, 24^3 x 32 186 -> 223)
-  a.per = g.V <= SPLIT_MAX_SITES ? 1 : a.nperm;
+  a.per = g.V <= WLOOP_ROW_SITES ? 1 : a.nperm;
   const int rows = (a.nperm + a.per - 1) / a.per;
   int r;
   if ((r = ensure_part(c, (size_t)nb * rows))) return r;
