@@ -16,12 +16,19 @@
 
 namespace mag {
 
-struct RecCall {
-  const void* kb = nullptr;  // batched kernel entry, void(*)(const A*)
+// A batched kernel, void(*)(const A*), and its launch for one chain.
+struct BatchKernel {
+  const void* k = nullptr;
   dim3 grid, block;
+};
+
+struct RecCall {
+  BatchKernel few, many;  // for fewer than many_from chains, for that many and more
+  int many_from = 0;      // 0: `few` for any number
   size_t argsz = 0;
   std::vector<char> blob;  // argsz bytes per recorded chain
   void* table = nullptr;   // device copy of blob (set when the plan is built)
+  const BatchKernel& kernel(size_t chains) const { return many_from && (int)chains >= many_from ? many : few; }
 };
 
 struct Recorder {
@@ -33,16 +40,16 @@ struct Recorder {
     chain = i;
     pos = 0;
   }
-  void add(const void* kb, dim3 grid, dim3 block, const void* args, size_t argsz) {
+  void add(const BatchKernel& few, const BatchKernel& many, int many_from, const void* args, size_t argsz) {
     if (chain == 0) {
       RecCall c;
-      c.kb = kb;
-      c.grid = grid;
-      c.block = block;
+      c.few = few;
+      c.many = many;
+      c.many_from = many_from;
       c.argsz = argsz;
       calls.push_back(std::move(c));
-    } else if (pos >= calls.size() || calls[pos].kb != kb || calls[pos].argsz != argsz ||
-               calls[pos].grid.x != grid.x || calls[pos].grid.y != grid.y) {
+    } else if (pos >= calls.size() || calls[pos].few.k != few.k || calls[pos].argsz != argsz ||
+               calls[pos].few.grid.x != few.grid.x || calls[pos].few.grid.y != few.grid.y) {
       mismatch = true;
       return;
     }
@@ -55,9 +62,9 @@ struct Recorder {
 
 template <class A>
 int launch(mag_ctx c, const char* timer, void (*ks)(A), void (*kb)(const A*), dim3 grid, const A& a,
-           int block = BLOCK) {
+           int block = BLOCK, const BatchKernel& many = {}, int many_from = 0) {
   if (c->rec) {
-    c->rec->add((const void*)kb, grid, dim3(block), &a, sizeof(A));
+    c->rec->add({(const void*)kb, grid, dim3(block)}, many, many_from, &a, sizeof(A));
     return MAG_OK;
   }
   KTimer t(c, timer);
@@ -67,13 +74,16 @@ int launch(mag_ctx c, const char* timer, void (*ks)(A), void (*kb)(const A*), di
   return MAG_OK;
 }
 
-// A stencil kernel in its split form: one wavefront per plane, 64 sites per block.
+// A stencil kernel in its split form: one wavefront per plane, 64 sites per
+// block; `many` from many_from chains in a batch.
 template <class K>
 struct Stencil {};
 template <class A, class K>
-int launch_split(mag_ctx c, const char* timer, Stencil<K>, const Geom& g, const A& a) {
-  return launch(c, timer, k_split<K>, k_split_b<K>, grid_split(g), a, PLANE_THREADS);
+int launch_split(mag_ctx c, const char* timer, Stencil<K>, const Geom& g, const A& a, const BatchKernel& many = {},
+                 int many_from = 0) {
+  return launch(c, timer, k_split<K>, k_split_b<K>, grid_split(g), a, PLANE_THREADS, many, many_from);
 }
+
 // The split form up to a number of sites, else one thread per link (ks, kb).
 // Below the line one thread per link leaves most SIMDs with one wavefront or
 // none; above it all are busy either way, and two of three wavefronts idle
@@ -101,10 +111,25 @@ constexpr bool split_wins(int V) {
   if (!K::smears) return V <= 24576;
   return V <= 8192 || (V > 16384 && V <= SPLIT_MAX_SITES);
 }
+// A served batch fills the chip with lattices that do not alone: from this many
+// sites in all its launches go one thread per link, with the same bits (from two
+// chains on, so that a chain alone keeps the form of Chain.run). FP64 rectangles
+// stay split. Trajectories, split and one thread per link, against the kernels
+// of larger lattices: FP32 Iwasaki + 3-stout 8^4, 8 chains 1.08 and 0.98, 64 chains
+// 1.09 and 1.00; FP64 Wilson + 2-stout 8^4, 4 chains 1.13 and 1.04, 64 chains 1.07
+// and 0.99; below the line 8^4 FP32, 4 chains 0.82 and 1.04, FP64, 2 chains 0.79
+// and 1.05.
+template <class K>
+constexpr int unsplit_from(int V) {
+  const int sites = sizeof(typename K::Real) == sizeof(float) || !K::smears ? 32768 : 16384;
+  return (sites + V - 1) / V < 2 ? 2 : (sites + V - 1) / V;
+}
 template <class A, class K>
 int launch_stencil(mag_ctx c, const char* timer, void (*ks)(A), void (*kb)(const A*), Stencil<K> k, const Geom& g,
                    const A& a) {
-  if (split_wins<K>(g.V)) return launch_split(c, timer, k, g, a);
+  if (split_wins<K>(g.V))
+    return launch_split(c, timer, k, g, a, {(const void*)k_unsplit_b<K>, grid_stencil(g), dim3(BLOCK)},
+                        unsplit_from<K>(g.V));
   return launch(c, timer, ks, kb, grid_stencil(g), a);
 }
 

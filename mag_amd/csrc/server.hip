@@ -210,8 +210,9 @@ int build_batch(mag_server s, Batch* b) {
   if (s->graphs) {
     HIPCHK(x, hipStreamBeginCapture(s->aux, hipStreamCaptureModeThreadLocal));
     for (auto& c : b->rec.calls) {
+      const BatchKernel& k = c.kernel(n);
       void* args[] = {&c.table};
-      (void)hipLaunchKernel(c.kb, dim3(c.grid.x, c.grid.y, (unsigned)n), c.block, args, 0, s->aux);
+      (void)hipLaunchKernel(k.k, dim3(k.grid.x, k.grid.y, (unsigned)n), k.block, args, 0, s->aux);
     }
     HIPCHK(x, hipStreamEndCapture(s->aux, &b->graph));
     HIPCHK(x, hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
@@ -245,8 +246,9 @@ int launch_batch(mag_server s, Batch* b) {
     HIPCHK(x, hipGraphLaunch(b->exec, st));
   } else {
     for (auto& c : b->rec.calls) {
+      const BatchKernel& k = c.kernel(n);
       void* args[] = {&c.table};
-      HIPCHK(x, hipLaunchKernel(c.kb, dim3(c.grid.x, c.grid.y, (unsigned)n), c.block, args, 0, st));
+      HIPCHK(x, hipLaunchKernel(k.k, dim3(k.grid.x, k.grid.y, (unsigned)n), k.block, args, 0, st));
     }
   }
   HIPCHK(x, hipMemcpyAsync(b->h_gather, b->gather, n * S_COUNT * sizeof(double), hipMemcpyDeviceToHost, st));
