@@ -1232,12 +1232,14 @@ MAG_D double block_max(double v) {
 // XCDs in turn, so that neighbours along x1 and x2 meet in one L2 while the
 // XCDs stay close together in memory. Plaquette / rectangle sums, blocks dealt
 // one by one -> by 16: 24^3 x 32 136 -> 113 / 308 -> 256 us, 32^4 276 -> 248 /
-// 629 -> 554. (One run per XCD does as well at 24^3 x 32, but takes 300 us for
-// the plaquettes of 32^4; the plaquettes alone in 131 instead of 358 registers,
-// three wavefronts per SIMD, take 160-390 us: too many sites at a time for L2.)
+// 629 -> 554. Up to one block per CU they are dealt one by one: 16^4 calls with
+// the sums read back, 12-real links 30.6 / 49.4 us, in runs 33.5 / 51.4. (One run
+// per XCD does as well at 24^3 x 32, but takes 300 us for the plaquettes of 32^4;
+// the plaquettes alone in 131 instead of 358 registers, three wavefronts per
+// SIMD, take 160-390 us: too many sites at a time for L2.)
 MAG_HD int run_block(int b, int nb) {
   constexpr int RUN = 16;
-  if (b >= nb / (8 * RUN) * (8 * RUN)) return b;
+  if (nb <= 256 || b >= nb / (8 * RUN) * (8 * RUN)) return b;
   const int j = b / 8;
   return (j / RUN) * 8 * RUN + (b % 8) * RUN + j % RUN;
 }

@@ -1,0 +1,33 @@
+// Host-side check of the walks that deal site blocks to the XCDs (kernels.hpp):
+// run_block (plaquette and rectangle sums) must be a permutation of the blocks,
+// and the identity up to one block per CU. One line per check; exits non-zero on
+// the first violation.
+#include <cstdio>
+#include <vector>
+
+#include "../../mag_amd/csrc/kernels.hpp"
+
+using namespace mag;
+
+template <class Map>
+static int permutation(const char* what, int nb, Map map) {
+  std::vector<int> hit((size_t)nb, 0);
+  for (int b = 0; b < nb; ++b) {
+    const int t = map(b);
+    if (t < 0 || t >= nb) return std::printf("FAIL %s: block %d of %d -> %d\n", what, b, nb, t), 1;
+    ++hit[(size_t)t];
+  }
+  for (int t = 0; t < nb; ++t)
+    if (hit[(size_t)t] != 1) return std::printf("FAIL %s: block %d of %d hit %d times\n", what, t, nb, hit[(size_t)t]), 1;
+  return 0;
+}
+
+int main() {
+  for (int nb = 1; nb < 1300; ++nb) {
+    if (permutation("run_block", nb, [&](int b) { return run_block(b, nb); })) return 1;
+    for (int b = 0; nb <= 256 && b < nb; ++b)
+      if (run_block(b, nb) != b) return std::printf("FAIL run_block: %d of %d moved\n", b, nb), 1;
+  }
+  std::printf("ok run_block\n");
+  return 0;
+}
