@@ -1413,11 +1413,16 @@ constexpr int WLOOP_ROW_SITES = 1 << 15;
 // Block of WLOOP_SITES sites that block b of nb takes: XCD k (b mod 8) has a
 // contiguous run of a walk with x3 fastest where an x3 slice is whole blocks
 // (the temporal lines of the sites that share them then meet in its L2: 24^3 x
-// 32, R = T = 4, 185 -> 151 us), else in site order.
+// 32, R = T = 4, 185 -> 151 us), else in site order. Of more than 32 slices x3
+// goes over eight at a time: with all 64 of 32^3 x 64 in flight the spatial
+// lines find nothing of the rows before (R = 4, T = 1, 657 us; by eights 590).
 MAG_HD int wloop_block(const Geom& g, int b, int nb) {
   const int k = b % 8, r = nb % 8;
   const int t = k * (nb / 8) + (k < r ? k : r) + b / 8;
-  return g.S[3] % WLOOP_SITES == 0 ? (t % g.L[3]) * (g.S[3] / WLOOP_SITES) + t / g.L[3] : t;
+  if (g.S[3] % WLOOP_SITES != 0) return t;
+  const int sb = g.S[3] / WLOOP_SITES, W = g.L[3] > 32 ? 8 : g.L[3];
+  const int w0 = t / (W * sb), i = t - w0 * W * sb, w = g.L[3] - W * w0 < W ? g.L[3] - W * w0 : W;
+  return (W * w0 + i % w) * sb + i / w;
 }
 
 MAG_D void site_step(const Geom& g, Site& y, int d) {
@@ -1496,6 +1501,41 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(TS
   }
   const double sum = block_sum(s < a.g.V ? acc : 0.);
   if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blk] = sum;
+}
+
+// The same with one thread per loop, every link in turn: fewer registers (129
+// against 180 on FP64 12-real links), so another wavefront per SIMD has its loads
+// in flight, which short loops on lattices beyond the last-level cache need more
+// than a shorter chain. The line between the two is wloop_short (ops_impl.hpp).
+template <class TS, int NC>
+__global__ __launch_bounds__(BLOCK) void k_wilson_loop_short(LinkView<TS, NC> U, WloopArgs a, double* part) {
+  const int s = blockIdx.x * BLOCK + threadIdx.x;
+  double acc = 0.;
+  if (s < a.g.V) {
+    for (int q = 0; q < a.nperm; ++q) {
+      Site y = site_of(a.g, s);
+      M3<double> m = unit3<double>();
+      auto fwd = [&](int d) {
+        m = mul(m, U.template load<double>(d, y.s));
+        y.s += off_rt(a.g, y, d, 1);
+        y.x[d] = (y.x[d] + 1 == a.g.L[d]) ? 0 : y.x[d] + 1;
+      };
+      auto bwd = [&](int d) {
+        y.s += off_rt(a.g, y, d, -1);
+        y.x[d] = (y.x[d] == 0) ? a.g.L[d] - 1 : y.x[d] - 1;
+        m = mul_nd(m, U.template load<double>(d, y.s));
+      };
+      for (int i = 0; i < 3; ++i)
+        for (int j = 0; j < a.r[q][i]; ++j) fwd(i);
+      for (int j = 0; j < a.T; ++j) fwd(3);
+      for (int i = 2; i >= 0; --i)
+        for (int j = 0; j < a.r[q][i]; ++j) bwd(i);
+      for (int j = 0; j < a.T; ++j) bwd(3);
+      acc += retrace(m);
+    }
+  }
+  const double t = block_sum(acc);
+  if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
 // Final reduction of block partials, one block, fixed order: each thread

@@ -362,6 +362,27 @@ int Ops<TS, NC>::unit(mag_ctx c, const Geom& g, void* U) {
   return MAG_OK;
 }
 
+// Whether loops of spatial extents r (ascending) by T go one thread per loop.
+// Calls with the sum read back, two wavefronts per loop over one thread per loop:
+//   r = 0, T = 1 / 2                   20^4 1.04 / 1.00, 24^3 x 32 1.13 / 1.04, 32^4 1.18 / 1.20
+//   FP32 R = T = 1                     24^4 0.97, 24^3 x 32 1.03, 28^4 1.03, 32^4 1.06
+//   FP32 (2,0,0) / (1,1,0), T = 1      24^3 x 32 1.00 / 0.94, 32^4 1.01 / 1.02, 48^2 x 16 x 32 1.03 / 1.03
+//   FP32 (1,1,1), T = 1 / 2 / 4        28^4 1.00 / 0.97 / 0.93, 32^4 1.12 / 1.09 / 1.05, 16^3 x 64 1.07 / 1.07 / 1.04
+//   FP64 12 reals, R = 1 / 2 / 4, T = 1  28^4 0.84 / 0.82 / 0.79, 32^4 1.09 / 1.11 / 1.03
+//   FP64 12 reals, (1,1,1), T = 2      32^4 0.89, 48^2 x 16 x 32 1.03, 32^3 x 48 1.07, 32^3 x 64 1.10
+// and at 32^4 FP32 R = 4, T = 1 0.97, R = T = 2 0.92, FP64 18 reals R = T = 1 0.85.
+template <class TS, int NC>
+bool wloop_short(const Geom& g, const int r[3], int nperm, int T) {
+  const long len = (long)r[0] + r[1] + r[2];
+  const int V = g.V;
+  if (len == 0) return T <= 2 && V > WLOOP_ROW_SITES;
+  if (NC != 12) return false;
+  if (std::is_same<TS, double>::value)
+    return (V > 3 << 18 && T == 1 && r[1] == 0) || (V > 5 << 18 && nperm == 1 && len <= 6);
+  return (V > 3 << 17 && len == 1 && T == 1) || (V > 3 << 18 && len <= 2 && T == 1) ||
+         (len == 3 && nperm == 1 && (V > 3 << 18 || (V > WLOOP_ROW_SITES && g.L[3] > 32)));
+}
+
 template <class TS, int NC>
 int Ops<TS, NC>::wilson_loop(mag_ctx c, const Geom& g, void* U, const int r3[3], int T, int slot, int* nperm) {
   WloopArgs a{};
@@ -374,12 +395,24 @@ int Ops<TS, NC>::wilson_loop(mag_ctx c, const Geom& g, void* U, const int r3[3],
     for (int i = 0; i < 3; ++i) a.r[a.nperm][i] = rl[i];
     a.nperm++;
   } while (std::next_permutation(rl, rl + 3));
+  *nperm = a.nperm;
+  int r;
+  if (wloop_short<TS, NC>(g, rl, a.nperm, T)) {
+    const int nb = (g.V + BLOCK - 1) / BLOCK;
+    if ((r = ensure_part(c, (size_t)nb))) return r;
+    {
+      KTimer t(c, "wilson_loop");
+      hipLaunchKernelGGL((k_wilson_loop_short<TS, NC>), dim3(nb), dim3(BLOCK), 0, c->stream, lview<TS, NC>(U, g), a,
+                         c->d_part);
+    }
+    CHECK_LAUNCH(c);
+    return final_reduce(c, c->d_part, nb, 1, 0, slot);
+  }
   const int nb = (g.V + WLOOP_SITES - 1) / WLOOP_SITES;
   // a row of the grid per permutation where the sites alone leave SIMDs idle
   // (R = T = 4: 8^4 15 -> 9 us, 12^4 17 -> 13; 16^4 27 -> 29, 24^3 x 32 186 -> 223)
   a.per = g.V <= WLOOP_ROW_SITES ? 1 : a.nperm;
   const int rows = (a.nperm + a.per - 1) / a.per;
-  int r;
   if ((r = ensure_part(c, (size_t)nb * rows))) return r;
   {
     KTimer t(c, "wilson_loop");
@@ -387,7 +420,6 @@ int Ops<TS, NC>::wilson_loop(mag_ctx c, const Geom& g, void* U, const int r3[3],
                        c->d_part);
   }
   CHECK_LAUNCH(c);
-  *nperm = a.nperm;
   return final_reduce(c, c->d_part, nb * rows, 1, 0, slot);
 }
 

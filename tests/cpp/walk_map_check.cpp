@@ -1,7 +1,8 @@
 // Host-side check of the walks that deal site blocks to the XCDs (kernels.hpp):
 // run_block (plaquette and rectangle sums) must be a permutation of the blocks,
-// and the identity up to one block per CU. One line per check; exits non-zero on
-// the first violation.
+// and the identity up to one block per CU; wloop_block (Wilson loops) must be a
+// permutation on any lattice, x3 in one piece or by eights with a remainder. One
+// line per check; exits non-zero on the first violation.
 #include <cstdio>
 #include <vector>
 
@@ -29,5 +30,14 @@ int main() {
       if (run_block(b, nb) != b) return std::printf("FAIL run_block: %d of %d moved\n", b, nb), 1;
   }
   std::printf("ok run_block\n");
+  const int shapes[][4] = {{4, 4, 4, 4},    {5, 7, 4, 9},    {16, 16, 16, 8}, {8, 4, 4, 32},  {8, 4, 4, 33},
+                           {8, 16, 4, 37},  {16, 8, 4, 40},  {4, 4, 8, 71},   {24, 16, 8, 48}, {32, 32, 4, 64},
+                           {12, 12, 12, 48}, {8, 8, 6, 100}};
+  for (const auto& L : shapes) {
+    const Geom g = make_geom(L);
+    const int nb = (g.V + WLOOP_SITES - 1) / WLOOP_SITES;
+    if (permutation("wloop_block", nb, [&](int b) { return wloop_block(g, b, nb); })) return 1;
+  }
+  std::printf("ok wloop_block\n");
   return 0;
 }
