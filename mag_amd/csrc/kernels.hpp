@@ -53,13 +53,15 @@ constexpr int stencil_waves() { return sizeof(TC) == sizeof(float) ? 3 : 2; }
 // (FP64 trajectory 2.7 % faster; the forward kernel and FP32 keep the first
 // order). Otherwise XCD k takes tiles [k nb/8, (k+1) nb/8) in lexicographic
 // order. nb = blocks in the launch, b = this block; every (mu, sblk) of the
-// 4 V / BLOCK tiles comes out of exactly one b.
-template <bool X2_INNER = false, int BS = BLOCK>
+// 4 ceil(V / BLOCK) tiles comes out of exactly one b. nb may be rounded up
+// (grid_stencil): the surplus blocks come out with sblk past the last site block,
+// and a kernel returns for them before any load, store or barrier.
+template <bool X2_INNER = false>
 MAG_HD void tile_map(const Geom& g, int nb, int b, int& mu, int& sblk) {
   const int plane = g.L[0] * g.L[1];
   const int slice = plane * g.L[2];
-  const bool slab = nb % 8 == 0 && g.L[3] % 8 == 0 && nb == 4 * (g.V / BS) &&
-                    (X2_INNER ? plane % BS == 0 : slice % BS == 0);
+  const bool slab = nb % 8 == 0 && g.L[3] % 8 == 0 && nb == 4 * (g.V / BLOCK) &&
+                    (X2_INNER ? plane % BLOCK == 0 : slice % BLOCK == 0);
   if (slab) {
     const int xcd = b % 8, j = b / 8;
     const int h3 = g.L[3] / 8;
@@ -69,14 +71,14 @@ MAG_HD void tile_map(const Geom& g, int nb, int b, int& mu, int& sblk) {
     r /= h3;
     int bs;  // block within the x3 slice
     if (X2_INNER) {
-      const int nb01 = plane / BS;
+      const int nb01 = plane / BLOCK;
       const int x2 = r % g.L[2];
       bs = x2 * nb01 + r / g.L[2];
     } else {
       bs = r;
     }
     const int x3 = xcd * h3 + dx3;
-    sblk = x3 * (slice / BS) + bs;
+    sblk = x3 * (slice / BLOCK) + bs;
     return;
   }
   const int t = (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;

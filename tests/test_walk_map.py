@@ -17,4 +17,4 @@ def test_every_block_once(tmp_path):
                    check=True, capture_output=True, timeout=600)
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
-    assert r.stdout.split("\n")[:-1] == ["ok run_block", "ok wloop_block"]
+    assert r.stdout.split("\n")[:-1] == ["ok run_block", "ok wloop_block", "ok tile_map"]
