@@ -81,24 +81,30 @@ __global__ __launch_bounds__(TB) void k_to_host(TS* p, int V, int s0, int ns, do
   }
 }
 
-template <class TS, int NC, bool ALG>
+// AHEAD of a thread's nine loads over the link are on their way at a time.
+template <class TS, int NC, bool ALG, int AHEAD>
 __global__ __launch_bounds__(TB) void k_from_host(TS* p, int V, int s0, int ns, const double* in) {
   __shared__ double buf[64 * LROW];
   const int lane = threadIdx.x & 63, mu = threadIdx.x >> 6, b0 = blockIdx.x * 64;
   const int n2 = min(64, ns - b0) * (ROW / 2);
   const V2* src = (const V2*)(in + (size_t)b0 * ROW);
-  // all loads over the link on their way at once (one by one 6 us more per call: 4^4 links 26.8 -> 20.7)
   constexpr int PER = 64 * (ROW / 2) / TB;
-  V2 v[PER];
+#pragma unroll 1
+  for (int k0 = 0; k0 < PER; k0 += AHEAD) {
+    V2 v[AHEAD];
 #pragma unroll
-  for (int k = 0; k < PER; ++k)
-    if ((int)threadIdx.x + k * TB < n2) v[k] = src[threadIdx.x + k * TB];
+    for (int k = 0; k < AHEAD; ++k) {
+      const int i = threadIdx.x + (k0 + k) * TB;
+      if (i < n2) v[k] = src[i];
+    }
 #pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int i = threadIdx.x + k * TB, site = i / (ROW / 2), c = 2 * (i - site * (ROW / 2));
-    if (i >= n2) break;
-    buf[site * LROW + c] = v[k][0];
-    buf[site * LROW + c + 1] = v[k][1];
+    for (int k = 0; k < AHEAD; ++k) {
+      const int i = threadIdx.x + (k0 + k) * TB, site = i / (ROW / 2), c = 2 * (i - site * (ROW / 2));
+      if (i < n2) {
+        buf[site * LROW + c] = v[k][0];
+        buf[site * LROW + c + 1] = v[k][1];
+      }
+    }
   }
   __syncthreads();
   if (b0 + lane >= ns) return;
@@ -129,9 +135,14 @@ __global__ __launch_bounds__(TB) void k_real_from_host(double* p, int V, int s0,
   if (i < 4 * ns) p[(size_t)(i & 3) * V + s0 + (i >> 2)] = in[i];
 }
 
+// Up, a chunk of at most 16 blocks waits for the link's latency, so its threads ask
+// for all they need at once (4^4 links 27 -> 20.5 us, 8^4 115 -> 102); with more
+// blocks the link is busy anyway, and nine lines per thread out of order take it
+// longer (16^4 853 -> 1069 us, 24^3 x 32 5.2 -> 6.7 ms).
 template <class TS, int NC, bool ALG>
-const void* matrix_kernel(bool down) {
-  return down ? (const void*)k_to_host<TS, NC, ALG> : (const void*)k_from_host<TS, NC, ALG>;
+const void* matrix_kernel(bool down, int ns) {
+  if (down) return (const void*)k_to_host<TS, NC, ALG>;
+  return ns <= 16 * 64 ? (const void*)k_from_host<TS, NC, ALG, 9> : (const void*)k_from_host<TS, NC, ALG, 1>;
 }
 
 // Sites [s0, s0 + ns) of f to (from) a pinned slot. Answers with the launch's
@@ -145,9 +156,9 @@ hipError_t launch_chunk(mag_field f, bool down, int s0, int ns, double* slot) {
       k = down ? (const void*)k_real_to_host : (const void*)k_real_from_host;
       nb = (4 * ns + TB - 1) / TB;
       break;
-    case MAG_ALG8: k = f64 ? matrix_kernel<double, 8, true>(down) : matrix_kernel<float, 8, true>(down); break;
-    case MAG_LINK12: k = f64 ? matrix_kernel<double, 12, false>(down) : matrix_kernel<float, 12, false>(down); break;
-    default: k = matrix_kernel<double, 18, false>(down);  // MAG_LINK18 fields are FP64
+    case MAG_ALG8: k = f64 ? matrix_kernel<double, 8, true>(down, ns) : matrix_kernel<float, 8, true>(down, ns); break;
+    case MAG_LINK12: k = f64 ? matrix_kernel<double, 12, false>(down, ns) : matrix_kernel<float, 12, false>(down, ns); break;
+    default: k = matrix_kernel<double, 18, false>(down, ns);  // MAG_LINK18 fields are FP64
   }
   int V = f->g.V;
   void* args[] = {&f->p, &V, &s0, &ns, &slot};
