@@ -18,8 +18,8 @@
 // of the raw field took 309 / 269 ms for its FP64 links, 106 / 133 ms for the
 // FP32 links and 91 / 101 ms for the momenta.
 //
-// Momenta and one-real-per-link fields of few sites cross as they are stored and
-// are converted by the calling thread (convert_here).
+// Momenta and forces of few sites cross as they are stored and are converted by
+// the calling thread (convert_here).
 //
 // Conversions are the host's own arithmetic (no fused multiply-adds), so the
 // values are bitwise the same either way.
@@ -205,27 +205,27 @@ int need_stage(mag_ctx c, size_t bytes, size_t events) {
   return MAG_OK;
 }
 
-// Momenta, forces and one-real-per-link fields of few sites: the field as it is
-// stored through a pinned slot, converted by this thread. Their host layout has
-// up to 4.5 times the bytes, all of which the kernels move over the link, and a
-// launch and an event cost as much as a small copy. Through the kernels -> here,
-// up / down (us):
-//   FP32 momenta  4^4 20.6 / 21.6 -> 14.6 / 15.1, 8^4 102 / 104 -> 60 / 63, 13,824 sites 249 / 260 -> 169 / 190
-//   FP64 momenta  4^4 20.9 / 21.8 -> 14.8 / 18.3, 8^4 104 / 104 -> 67 / 99, 6,144 sites 139 / 145 -> 91 / 160
-//   one real      6^4 17.4 / 17.0 -> 12.8 / 13.5, 8^4 19.6 / 20.2 -> 15.4 / 17.1, 13,824 sites 30 / 33 -> 27 / 33
-// Links go through the kernels from 4^4 on.
-constexpr int HERE_SITES = 16384, HERE_SITES_ALG64 = 4096;
+// Momenta and forces of few sites: the field as it is stored through a pinned
+// slot, converted by this thread. Their host layout has 2.25 (FP64) or 4.5 times
+// the bytes, all of which the conversion kernels move over the link. Behind a force
+// kernel, through those kernels -> here, up / down:
+//   FP32  4^4 30 / 25 -> 22 / 22 us, 6^4 57 / 49 -> 32 / 31, 8^4 118 / 107 -> 63 / 58, 13,824 sites 248 / 264 -> 170 / 152
+//   FP64  4^4 30 / 25 -> 22 / 24, 6^4 57 / 49 -> 37 / 38, 8^4 122 / 105 -> 79 / 108
+// Links and one real per link gain nothing here.
+constexpr int HERE_SITES32 = 16384, HERE_SITES64 = 4096;
 bool convert_here(mag_field f) {
-  if (f->kind == MAG_REAL1) return f->g.V <= HERE_SITES;
-  return f->kind == MAG_ALG8 && f->g.V <= (f->prec == MAG_F64 ? HERE_SITES_ALG64 : HERE_SITES);
+  return f->kind == MAG_ALG8 && f->g.V <= (f->prec == MAG_F64 ? HERE_SITES64 : HERE_SITES32);
 }
 template <class TS>
 void alg_here(TS* raw, double* host, int V, bool down) {
   constexpr int W = Packed<TS, 8>::W, NG = 8 / W;
-  constexpr int RUN = 32;  // sites at a time by direction: the groups of all four directions would share cache sets
-  for (int s0 = 0; s0 < V; s0 += RUN)
+  // FP64: 32 sites at a time by direction, where the sixteen groups of all four
+  // directions would share cache sets (8^4 down 100 -> 77 us; 6^4, whose groups
+  // do not, 29 site by site and 40 so)
+  const int run = NG == 2 || (down && (size_t)V * W * sizeof(TS) % 4096 != 0) ? 1 : 32;
+  for (int s0 = 0; s0 < V; s0 += run)
     for (int mu = 0; mu < 4; ++mu)
-      for (int s = s0; s < std::min(s0 + RUN, V); ++s) {
+      for (int s = s0; s < std::min(s0 + run, V); ++s) {
         double* m = host + ((size_t)s * 4 + mu) * 18;
         TS* r = raw + ((size_t)mu * NG * V + s) * W;
         const size_t group = (size_t)V * W;
@@ -245,26 +245,26 @@ void alg_here(TS* raw, double* host, int V, bool down) {
         }
       }
 }
-void real_here(double* raw, double* host, int V, bool down) {
-  for (int s = 0; s < V; ++s)
-    for (int mu = 0; mu < 4; ++mu) {
-      double &r = raw[(size_t)mu * V + s], &h = host[(size_t)s * 4 + mu];
-      if (down) h = r;
-      else r = h;
-    }
+// A kernel, not the copy engine: alone that is 3 us faster, but behind work still in
+// flight, as a result that is read back, it is 7 us slower (it waits in a queue of
+// its own).
+__global__ __launch_bounds__(TB) void k_raw(const V2* src, V2* dst, int n) {
+  const int i = blockIdx.x * TB + threadIdx.x;
+  if (i < n) dst[i] = src[i];
 }
 int transfer_raw(mag_field f, double* host, bool down) {
   mag_ctx c = f->ctx;
   int r;
   if ((r = need_stage(c, f->bytes, 0))) return r;
   auto convert = [&] {
-    if (f->kind == MAG_REAL1) real_here((double*)c->stage, host, f->g.V, down);
-    else if (f->prec == MAG_F64) alg_here((double*)c->stage, host, f->g.V, down);
+    if (f->prec == MAG_F64) alg_here((double*)c->stage, host, f->g.V, down);
     else alg_here((float*)c->stage, host, f->g.V, down);
   };
   if (!down) convert();
-  HIPCHK(c, down ? hipMemcpyAsync(c->stage, f->p, f->bytes, hipMemcpyDeviceToHost, c->stream)
-                 : hipMemcpyAsync(f->p, c->stage, f->bytes, hipMemcpyHostToDevice, c->stream));
+  int n = (int)(f->bytes / sizeof(V2));  // whole: 32 V bytes or more
+  void *src = down ? f->p : c->stage, *dst = down ? c->stage : f->p;
+  void* args[] = {&src, &dst, &n};
+  HIPCHK(c, hipLaunchKernel((const void*)k_raw, dim3((n + TB - 1) / TB), dim3(TB), args, 0, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (down) convert();
   return MAG_OK;

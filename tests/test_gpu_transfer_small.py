@@ -1,6 +1,6 @@
-"""Momenta and one-real-per-link fields on either side of the sizes up to which
-the calling thread converts them, and a lattice that leaves its last run of sites
-ragged: bit for bit the host arithmetic that both ways stand for."""
+"""Momenta on either side of the sizes up to which the calling thread converts
+them, a lattice that leaves its last run of sites ragged, and one-real-per-link
+fields of the same sizes: bit for bit the host arithmetic that both ways stand for."""
 import numpy as np
 import pytest
 
