@@ -501,6 +501,7 @@ template <int ACT, bool CONS, class TS, int NC, class TC>
 struct ForceStencil {
   using Args = ForceArgs<TS, NC>;
   using Real = TC;
+  static constexpr int reals = NC;
   static constexpr bool smears = false;
   static constexpr int waves = stencil_waves<TC>();
   MAG_D static M3<TC> share(const Args& a, const Site& p, int mu, int plane) {

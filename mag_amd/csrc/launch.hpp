@@ -101,15 +101,17 @@ int launch_split(mag_ctx c, const char* timer, Stencil<K>, const Geom& g, const 
 //   FP64 thin, 12-real links      0.74    0.88    0.95    0.84    0.93    0.98    1.02    1.06
 // FP64 one thread per link takes as long for any lattice up to 16,384 sites (one
 // wavefront per SIMD) and nearly twice that from there; the split form, two blocks
-// per CU, needs a second round from 8,192. Six wavefronts (plane and side) took 50
-// us at FP32 8^4 but 149 at 12^4; three groups of sites per block, every wavefront
-// going on with one, gave the split's gain back.
+// per CU, needs a second round from 8,192, which costs it the gain by 12,288, and a
+// smearing by itself, without the backward kernels, already 4-9 % (smear() gives
+// split_max). Six wavefronts (plane and side) took 50 us at FP32 8^4 but 149 at
+// 12^4; three groups of sites per block, every wavefront going on with one, gave
+// the split's gain back.
 constexpr int SPLIT_MAX_SITES = 20736;  // 12^4
 template <class K>
 constexpr bool split_wins(int V) {
-  if (sizeof(typename K::Real) == sizeof(float)) return V <= SPLIT_MAX_SITES;
-  if (!K::smears) return V <= 24576;
-  return V <= 8192 || (V > 16384 && V <= SPLIT_MAX_SITES);
+  if constexpr (sizeof(typename K::Real) == sizeof(float)) return V <= SPLIT_MAX_SITES;
+  else if constexpr (!K::smears) return V <= (K::reals == 12 ? 24576 : 32768);
+  else return V <= 12288 || (V > 16384 && V <= SPLIT_MAX_SITES);
 }
 // A served batch fills the chip with lattices that do not alone: from this many
 // sites in all its launches go one thread per link, with the same bits (from two
@@ -126,8 +128,8 @@ constexpr int unsplit_from(int V) {
 }
 template <class A, class K>
 int launch_stencil(mag_ctx c, const char* timer, void (*ks)(A), void (*kb)(const A*), Stencil<K> k, const Geom& g,
-                   const A& a) {
-  if (split_wins<K>(g.V))
+                   const A& a, int split_max = SPLIT_MAX_SITES) {
+  if (split_wins<K>(g.V) && (!K::smears || g.V <= split_max))
     return launch_split(c, timer, k, g, a, {(const void*)k_unsplit_b<K>, grid_stencil(g), dim3(BLOCK)},
                         unsplit_from<K>(g.V));
   return launch(c, timer, ks, kb, grid_stencil(g), a);

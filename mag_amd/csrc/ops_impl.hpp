@@ -59,19 +59,16 @@ int Ops<TS, NC>::link_update(mag_ctx c, const Geom& g, void* Uin, void* Uout, vo
 // = 2: 4^4 58 -> 22 us, 8^4 61 -> 24, 12^4 107 -> 60; FP32 61 -> 17, 65 -> 18,
 // 64 -> 27). On larger lattices that costs little, and those blocks, which
 // share no neighbours with the stencil's in flight, cost more: 32^4 2.44 ms in
-// one thread per link, 2.86 with them; FP64 Wilson at 28,672 sites 1.08 of one
-// thread per link (at 27,648 0.98). Block size 1 has no such link and no force at
-// all (the classes alone say so: 5 us against 45 at 12^4), and a negative size,
+// one thread per link, 2.86 with them; at 32,768 sites FP64 Wilson 29 -> 25 us (16^3
+// x 8; 8 x 14 x 16^2 19 -> 21), Iwasaki 121 -> 77. Block size 1 has no such link and no
+// force at all (the classes alone say so: 5 us against 45 at 12^4), and a negative size,
 // whose links are never the last of a block, is not one that pair_site lists.
-template <int ACT, class TS>
-bool gather_pairs(const Geom& g, int mag) {
-  return mag >= 2 && g.V <= (ACT == ACT_WILSON && std::is_same<TS, double>::value ? 24576 : 32768);
-}
+inline bool gather_pairs(const Geom& g, int mag) { return mag >= 2 && g.V <= 32768; }
 template <int ACT, class TS, int NC>
 int thin_force(mag_ctx c, ForceArgs<TS, NC> fa) {
   const char* name = ACT == ACT_IWASAKI ? "force_iwasaki" : "force_wilson";
   const Geom& g = fa.g;
-  if (fa.mag && !gather_pairs<ACT, TS>(g, fa.mag))
+  if (fa.mag && !gather_pairs(g, fa.mag))
     return launch(c, name, k_gauge_force<ACT, true, TS, NC, TS>, k_gauge_force_b<ACT, true, TS, NC, TS>,
                   grid_stencil(g), fa);
   if (fa.mag) {
@@ -319,7 +316,8 @@ int Ops<TS, NC>::smear(mag_ctx c, const Geom& g, void* Uout, void* U, double rho
     StoutFwdArgs<TS, NC, TS, NC> fw{g, lview<TS, NC>(src, g), aview<TS>(nullptr, g), mview<TS>(nullptr, g),
                                     lview<TS, NC>(dst, g), rho, 0};
     if ((r = launch_stencil(c, "stout_fwd", k_stout_fwd<TS, NC, TS, NC, TS>, k_stout_fwd_b<TS, NC, TS, NC, TS>,
-                            Stencil<FwdStencil<TS, NC, TS, NC, TS>>{}, g, fw)))
+                            Stencil<FwdStencil<TS, NC, TS, NC, TS>>{}, g, fw,
+                            std::is_same<TS, double>::value ? 8192 : SPLIT_MAX_SITES)))
       return r;
     src = dst;
   }
