@@ -117,13 +117,13 @@ constexpr bool split_wins(int V) {
 // sites in all its launches go one thread per link, with the same bits (from two
 // chains on, so that a chain alone keeps the form of Chain.run). FP64 rectangles
 // stay split. Trajectories, split and one thread per link, against the kernels
-// of larger lattices: FP32 Iwasaki + 3-stout 8^4, 8 chains 1.08 and 0.98, 64 chains
-// 1.09 and 1.00; FP64 Wilson + 2-stout 8^4, 4 chains 1.13 and 1.04, 64 chains 1.07
-// and 0.99; below the line 8^4 FP32, 4 chains 0.82 and 1.04, FP64, 2 chains 0.79
-// and 1.05.
+// of larger lattices: FP32 Iwasaki + 3-stout, 16 chains of 6^4 (20,736 sites) 0.76
+// and 0.78, 7 of 8^4 (28,672) 1.11 split, 64 of 8^4 1.09 and 1.00; FP64 Wilson
+// + 2-stout 8^4, 2 chains 0.79 and 1.05, 4 chains 1.13 and 1.04, 64 chains 1.07 and
+// 0.99.
 template <class K>
 constexpr int unsplit_from(int V) {
-  const int sites = sizeof(typename K::Real) == sizeof(float) || !K::smears ? 32768 : 16384;
+  const int sites = sizeof(typename K::Real) == sizeof(float) || !K::smears ? 24576 : 16384;
   return (sites + V - 1) / V < 2 ? 2 : (sites + V - 1) / V;
 }
 template <class A, class K>
