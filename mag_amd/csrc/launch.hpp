@@ -3,9 +3,9 @@
 // on the context stream; with a recorder attached (serving, see server.hip)
 // it records the call instead. A batch of chains of one shape class records
 // the same call sequence once per chain; the recorder then emits one launch
-// per call of the batched kernel variant, whose argument table holds one
-// entry per chain (blockIdx.z = chain). The emitted sequence has fixed
-// arguments, so it can be captured in a HIP graph and replayed.
+// per call of the batched kernel variant (of two, the one for the number of
+// chains), whose argument table holds one entry per chain. The emitted sequence
+// has fixed arguments, so it can be captured in a HIP graph and replayed.
 #pragma once
 #include <cstring>
 #include <string>

@@ -29,8 +29,9 @@
 //     their memory returns to the budget once the device is done with it.
 // mag_server_step() admits, launches every idle batch, then waits until at
 // least one batch in flight has completed and processes all that have.
-// A chain's kernels and reductions are the same alone or in a batch, so its
-// results do not depend on what it is batched with or when.
+// A chain's sums and reductions are the same alone or in a batch (a large batch
+// may run its stencils in another form, with the same sums in the same order), so
+// its results do not depend on what it is batched with or when.
 #include <chrono>
 #include <cmath>
 #include <cstring>
